@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <cstring>
 #include <map>
 #include <stdexcept>
 #include <string>
@@ -63,6 +64,8 @@ struct DevCtl {
     double stress_kin[6]; // last kinetic stress sum m v_a v_b (eV, Voigt xx yy zz xy xz yz)
     int steps_done;       // steps of the current run completed (advanced by the end-of-step kernel)
     double red[6];        // fixed-order sums of the last NoseHooverNPT reduction
+    int fill_halo;        // fullest halo and brick of the last unconditional list build
+    int fill_atoms;
 };
 
 // A rebuild that overflowed the neighbor capacity or a brick halo leaves the
@@ -93,6 +96,10 @@ struct atvh_ctx {
     std::string timing_only; // empty: every kernel family
     std::map<std::string, atvh::TimerSlot> timers;
     std::vector<hipEvent_t> event_pool;
+    // pinned host staging of this context (one host thread at a time; every
+    // user drains the stream before it returns), at most kPinMax bytes
+    void* pin = nullptr;
+    size_t pin_bytes = 0;
 };
 
 struct atvh_system {
@@ -101,7 +108,12 @@ struct atvh_system {
     int64_t npad = 0; // column stride of the ELL neighbor list
     double box[3] = {0, 0, 0};
 
-    // per-atom device arrays, cell-sorted order
+    // per-atom device arrays, cell-sorted order. The FP64 columns are one
+    // allocation of columns `col` doubles apart, in the order declared here
+    // (state, permutation scratch, x_save), the int columns another.
+    int64_t col = 0;
+    double* slab = nullptr;
+    int* islab = nullptr;
     double *x = nullptr, *y = nullptr, *z = nullptr;
     double *vx = nullptr, *vy = nullptr, *vz = nullptr;
     double *fx = nullptr, *fy = nullptr, *fz = nullptr;
@@ -145,6 +157,7 @@ struct atvh_system {
     int* perm = nullptr;
     int* scan_sums = nullptr;
     int nscan_blocks = 0;
+    std::vector<int> nl_sig; // grid, bricks and stencil the list's tables were made for
     int* nbr = nullptr;      // small-grid mode: ELL, column-major: nbr[k*npad + i]
     int* numneigh = nullptr; // [n]
     int cap = 0;
@@ -210,6 +223,8 @@ struct BatchStage {
     int nblocks = 0;
     int nmembers = 0; // entries of args (base holds nmembers + 1): the member search's range
     int* owner = nullptr; // [nblocks] member of every block (one load instead of a search)
+    std::vector<char> raw;   // host copy of args and the block counts they were built with
+    std::vector<int> blocks;
 };
 
 struct atvh_batch {
@@ -222,6 +237,8 @@ struct atvh_batch {
     unsigned char* nl_flags = nullptr; // [nsys] this step's rebuild flags
     int* nl_next = nullptr;            // work counter of the pair-build stage (k_batched_queue)
     bool typed = false;
+    bool stages_changed = false; // some stage's tables were re-made (a captured step is stale)
+    std::vector<int> nl_blocks;  // host copy of nl_nb
     // members whose force call is not the batched PairLJCut stage (charged
     // LJ + Coulomb with or without PME): queued one by one inside the step
     std::vector<atvh_system*> solo;
@@ -246,6 +263,26 @@ inline int grid_capped(int64_t n, int block = kBlock) {
     int g = grid_for(n, block);
     return g > kMaxGrid ? kMaxGrid : g;
 }
+
+// Pinned staging buffer of at least `bytes` (<= kPinMax); contents are the
+// caller's until its next stream synchronisation.
+constexpr size_t kPinMax = size_t(16) << 20;
+constexpr size_t kPinMin = size_t(256) << 10; // held from the context's creation
+void* ctx_pin(atvh_ctx* c, size_t bytes);
+// The control block as of everything queued so far: one asynchronous copy into
+// pinned memory and one stream synchronisation.
+void read_ctl(atvh_system* s, DevCtl& h);
+// Device arrays into host arrays, queued together, one synchronisation.
+struct HostPiece {
+    void* dst;
+    const void* src;
+    size_t bytes;
+};
+// Frames of up to this many staged bytes travel through the context's pinned
+// buffer (one copy each way, one synchronisation); larger ones column by
+// column from and to the caller's memory, where the copy itself is the cost.
+constexpr size_t kStageMax = size_t(8) << 20;
+void fetch_pieces(atvh_ctx* c, const std::vector<HostPiece>& pieces);
 
 // Timing helpers (HIP events on the context stream, around one kernel family).
 struct ScopedTimer {
@@ -374,10 +411,20 @@ void energy_enqueue_finalize(atvh_system* s, double* record_pe, int step, bool w
 
 namespace atvh {
 
+// The stage's device tables; a stage whose argument blocks and block counts
+// are those of the last run keeps them (a batch advances chunk after chunk
+// with unchanged members: re-making twelve stages took ~2 ms a run).
 template <class Args>
 void batch_stage(atvh_batch* b, const std::string& name, const std::vector<Args>& args,
                  const std::vector<int>& blocks) {
     BatchStage& st = b->stages[name];
+    const char* raw = reinterpret_cast<const char*>(args.data());
+    const size_t nraw = args.size() * sizeof(Args);
+    if (st.args && st.blocks == blocks && st.raw.size() == nraw && std::memcmp(st.raw.data(), raw, nraw) == 0)
+        return;
+    b->stages_changed = true;
+    st.raw.assign(raw, raw + nraw);
+    st.blocks = blocks;
     dev_free(st.args);
     dev_free(st.base);
     dev_free(st.owner);

@@ -147,11 +147,15 @@ void build_stages(atvh_batch* b, int nsteps) {
             s->d_thermo, nrec);
         ATVH_HIP(hipGetLastError());
     }
-    batch_free_stages(b);
-    free_graphs(b);
+    // stages whose members' arguments are unchanged keep their tables, and
+    // the captured step stays valid with them; a step that queues a member's
+    // own force call captures that call's arguments, so it is captured anew
+    b->stages_changed = false;
     integ_batch_build(b);
     nl_batch_build(b);
     pair_batch_build(b);
+    if (b->stages_changed || !b->solo.empty())
+        free_graphs(b);
 }
 
 } // namespace
@@ -332,8 +336,7 @@ int atvh_batch_run(atvh_batch* b, int nsteps, int precision, int energy_every) {
     k_batch_halted<<<(nsys + kBlock - 1) / kBlock, kBlock, 0, st>>>(b->d_ctls, nsys, b->d_halted);
     ATVH_HIP(hipGetLastError());
     std::vector<int> halted_h(nsys);
-    ATVH_HIP(hipStreamSynchronize(st));
-    ATVH_HIP(hipMemcpy(halted_h.data(), b->d_halted, nsys * sizeof(int), hipMemcpyDeviceToHost));
+    fetch_pieces(c, {HostPiece{halted_h.data(), b->d_halted, nsys * sizeof(int)}});
     for (int k = 0; k < nsys; ++k)
         if (halted_h[k])
             md_recover_and_finish(b->sys[k], nsteps, precision, energy_every);

@@ -1801,9 +1801,8 @@ int atvh_pme_info(atvh_system* s, int* K, double* e_parts) {
         for (int d = 0; d < 3; ++d)
             K[d] = s->pme->K[d];
     if (e_parts) {
-        ATVH_HIP(hipStreamSynchronize(c->stream));
         DevCtl h;
-        ATVH_HIP(hipMemcpy(&h, s->ctl, sizeof(h), hipMemcpyDeviceToHost));
+        read_ctl(s, h);
         for (int k = 0; k < 3; ++k)
             e_parts[k] = h.e_kspace[k];
     }

@@ -43,6 +43,72 @@ ScopedTimer::~ScopedTimer() {
         ctx->timers[name].pending.emplace_back(start, stop);
 }
 
+void* ctx_pin(atvh_ctx* c, size_t bytes) {
+    if (bytes > kPinMax)
+        throw Error(ATVH_E_ARG, "staging request beyond the pinned buffer's bound");
+    if (bytes > c->pin_bytes) {
+        if (c->pin)
+            (void)hipHostFree(c->pin);
+        c->pin = nullptr;
+        c->pin_bytes = 0;
+        size_t want = kPinMin;
+        while (want < bytes)
+            want *= 2;
+        if (hipHostMalloc(&c->pin, want, hipHostMallocDefault) != hipSuccess) {
+            c->pin = nullptr;
+            throw Error(ATVH_E_NOMEM, "hipHostMalloc of the staging buffer failed");
+        }
+        c->pin_bytes = want;
+    }
+    return c->pin;
+}
+
+void read_ctl(atvh_system* s, DevCtl& h) {
+    atvh_ctx* c = s->ctx;
+    void* p = ctx_pin(c, sizeof(DevCtl));
+    ATVH_HIP(hipMemcpyAsync(p, s->ctl, sizeof(DevCtl), hipMemcpyDeviceToHost, c->stream));
+    ATVH_HIP(hipStreamSynchronize(c->stream));
+    std::memcpy(&h, p, sizeof(DevCtl));
+}
+
+void fetch_pieces(atvh_ctx* c, const std::vector<HostPiece>& pieces) {
+    // pieces that follow each other on the device (columns of one allocation)
+    // leave as one copy; `at` is each piece's place in the pinned buffer
+    auto up = [](size_t b) { return (b + 511) & ~size_t(511); };
+    struct Run {
+        const char* src;
+        size_t bytes, at;
+    };
+    std::vector<Run> runs;
+    std::vector<size_t> at;
+    size_t total = 0;
+    for (const HostPiece& q : pieces) {
+        const char* src = static_cast<const char*>(q.src);
+        if (!runs.empty() && runs.back().src + up(runs.back().bytes) == src) {
+            at.push_back(runs.back().at + (src - runs.back().src));
+            runs.back().bytes = (src - runs.back().src) + q.bytes;
+        } else {
+            if (!runs.empty())
+                total = runs.back().at + up(runs.back().bytes);
+            runs.push_back(Run{src, q.bytes, total});
+            at.push_back(total);
+        }
+        total = runs.back().at + up(runs.back().bytes);
+    }
+    if (total > kStageMax) {
+        for (const HostPiece& q : pieces)
+            ATVH_HIP(hipMemcpyAsync(q.dst, q.src, q.bytes, hipMemcpyDeviceToHost, c->stream));
+        ATVH_HIP(hipStreamSynchronize(c->stream));
+        return;
+    }
+    char* pin = static_cast<char*>(ctx_pin(c, total));
+    for (const Run& r : runs)
+        ATVH_HIP(hipMemcpyAsync(pin + r.at, r.src, r.bytes, hipMemcpyDeviceToHost, c->stream));
+    ATVH_HIP(hipStreamSynchronize(c->stream));
+    for (size_t k = 0; k < pieces.size(); ++k)
+        std::memcpy(pieces[k].dst, pin + at[k], pieces[k].bytes);
+}
+
 static void resolve_timers(atvh_ctx* c) {
     ATVH_HIP(hipStreamSynchronize(c->stream));
     for (auto& kv : c->timers) {
@@ -77,49 +143,48 @@ static void resolve_timers(atvh_ctx* c) {
 namespace {
 
 // Frame-order gather for downloads; positions are wrapped into [0, L) here
-// (wrap_orthorhombic, pbc.h:37-51), velocities get the pending NH scale.
-__global__ void k_gather_out(int64_t n, const int* __restrict__ tag, const double* __restrict__ a,
-                             const double* __restrict__ b, const double* __restrict__ c,
-                             double* __restrict__ oa, double* __restrict__ ob,
-                             double* __restrict__ oc, const DevCtl* ctl, int mode, double la,
-                             double lb, double lc) {
-    const double s = mode == 1 ? ctl->nh_scale : 1.0;
+// (wrap_orthorhombic, pbc.h:37-51), velocities get the pending NH scale. The
+// nine state columns are `col` apart from `in` on, their frame-order copies
+// from `out` on; groups: bit 0 positions, 1 velocities, 2 forces.
+__global__ void k_gather_out(int64_t n, int64_t col, const int* __restrict__ tag, const double* __restrict__ in,
+                             double* __restrict__ out, const DevCtl* ctl, int groups, double la, double lb,
+                             double lc) {
+    const double s = ctl->nh_scale;
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
          i += (int64_t)gridDim.x * blockDim.x) {
         const int t = tag[i];
-        double va = a[i], vb = b[i], vc = c[i];
-        if (mode == 1) {
-            va *= s;
-            vb *= s;
-            vc *= s;
-        } else if (mode == 2) {
-            va -= la * floor(va / la);
-            vb -= lb * floor(vb / lb);
-            vc -= lc * floor(vc / lc);
+        if (groups & 1) {
+            const double va = in[i], vb = in[col + i], vc = in[2 * col + i];
+            out[t] = va - la * floor(va / la);
+            out[col + t] = vb - lb * floor(vb / lb);
+            out[2 * col + t] = vc - lc * floor(vc / lc);
         }
-        oa[t] = va;
-        ob[t] = vb;
-        oc[t] = vc;
+        if (groups & 2)
+            for (int k = 3; k < 6; ++k)
+                out[k * col + t] = in[k * col + i] * s;
+        if (groups & 4)
+            for (int k = 6; k < 9; ++k)
+                out[k * col + t] = in[k * col + i];
     }
 }
 
-__global__ void k_iota(int64_t n, int* __restrict__ tag) {
+// A fresh frame: slots in frame order, no pending thermostat scale.
+__global__ void k_frame_reset(int64_t n, int* __restrict__ tag, DevCtl* ctl) {
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
          i += (int64_t)gridDim.x * blockDim.x)
         tag[i] = static_cast<int>(i);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        ctl->nh_scale = 1.0;
+        ctl->always = 1;
+    }
 }
 
+
 void sys_free_all(atvh_system* s) {
-    double** dptrs[] = {&s->x,  &s->y,  &s->z,  &s->vx,  &s->vy,  &s->vz,  &s->fx, &s->fy,
-                        &s->fz, &s->q,  &s->ax, &s->ay,  &s->az,  &s->avx, &s->avy, &s->avz,
-                        &s->afx, &s->afy, &s->afz, &s->aq, &s->xs, &s->ys, &s->zs, &s->partials,
-                        &s->d_thermo};
-    for (auto p : dptrs)
-        dev_free(*p);
-    dev_free(s->type);
-    dev_free(s->tag);
-    dev_free(s->atype);
-    dev_free(s->atag);
+    dev_free(s->slab);
+    dev_free(s->islab);
+    dev_free(s->partials);
+    dev_free(s->d_thermo);
     dev_free(s->ctl);
     nl_free(s);
     pair_free(s);
@@ -147,6 +212,7 @@ int atvh_ctx_create(int device, atvh_ctx** out) {
     c->stream = c->own_stream;
     try {
         noalloc_bind(device);
+        ctx_pin(c, kPinMin);
     } catch (const Error&) {
         (void)hipStreamDestroy(c->own_stream);
         delete c;
@@ -174,6 +240,8 @@ int atvh_ctx_destroy(atvh_ctx* c) {
         (void)hipEventDestroy(e);
     if (c->own_stream)
         (void)hipStreamDestroy(c->own_stream);
+    if (c->pin)
+        (void)hipHostFree(c->pin);
     delete c;
     return ATVH_OK;
 }
@@ -275,12 +343,15 @@ int atvh_system_create(atvh_ctx* c, int64_t n, const double box[3], atvh_system*
     double** arrs[] = {&s->x,  &s->y,  &s->z,   &s->vx,  &s->vy,  &s->vz,  &s->fx, &s->fy, &s->fz,
                        &s->q,  &s->ax, &s->ay,  &s->az,  &s->avx, &s->avy, &s->avz, &s->afx,
                        &s->afy, &s->afz, &s->aq, &s->xs, &s->ys, &s->zs};
-    for (auto p : arrs)
-        dev_alloc(p, n);
-    dev_alloc(&s->type, n);
-    dev_alloc(&s->tag, n);
-    dev_alloc(&s->atype, n);
-    dev_alloc(&s->atag, n);
+    s->col = s->npad;
+    constexpr int kCols = sizeof(arrs) / sizeof(arrs[0]);
+    dev_alloc(&s->slab, size_t(kCols) * s->col);
+    for (int k = 0; k < kCols; ++k)
+        *arrs[k] = s->slab + k * s->col;
+    int** iarrs[] = {&s->type, &s->tag, &s->atype, &s->atag};
+    dev_alloc(&s->islab, size_t(4) * s->col);
+    for (int k = 0; k < 4; ++k)
+        *iarrs[k] = s->islab + k * s->col;
     dev_alloc(&s->ctl, 1);
     s->npartials = kMaxGrid;
     dev_alloc(&s->partials, size_t(2 * s->npartials) * kPartialStride); // pair | kinetic
@@ -288,10 +359,9 @@ int atvh_system_create(atvh_ctx* c, int64_t n, const double box[3], atvh_system*
     h.nh_scale = 1.0;
     h.always = 1;
     ATVH_HIP(hipMemcpyAsync(s->ctl, &h, sizeof(h), hipMemcpyHostToDevice, c->stream));
-    for (auto p : arrs)
-        ATVH_HIP(hipMemsetAsync(*p, 0, n * sizeof(double), c->stream));
-    ATVH_HIP(hipMemsetAsync(s->type, 0, n * sizeof(int), c->stream));
-    k_iota<<<grid_capped(n), kBlock, 0, c->stream>>>(n, s->tag);
+    ATVH_HIP(hipMemsetAsync(s->slab, 0, size_t(kCols) * s->col * sizeof(double), c->stream));
+    ATVH_HIP(hipMemsetAsync(s->islab, 0, size_t(4) * s->col * sizeof(int), c->stream));
+    k_frame_reset<<<grid_capped(n), kBlock, 0, c->stream>>>(n, s->tag, s->ctl);
     ATVH_HIP(hipGetLastError());
     ATVH_HIP(hipStreamSynchronize(c->stream));
     c->live_systems += 1;
@@ -376,41 +446,78 @@ int atvh_frame_upload(atvh_system* s, const double* x, const double* y, const do
     int ntypes = 1;
     double mt[kMaxTypes];
     bool seen[kMaxTypes] = {false};
-    for (int64_t i = 0; i < n; ++i) {
-        const int t = type ? type[i] : 0;
-        if (t < 0 || t >= kMaxTypes)
-            throw Error(ATVH_E_ARG, "atvh_frame_upload: type out of range [0,16)");
-        if (!(mass[i] > 0.0))
-            throw Error(ATVH_E_ARG, "atvh_frame_upload: mass must be positive");
-        if (!seen[t]) {
-            seen[t] = true;
-            mt[t] = mass[i];
-        } else if (mt[t] != mass[i]) {
-            throw Error(ATVH_E_ARG, "atvh_frame_upload: atoms of one type must share one mass");
+    // the common frame (one type, one mass) is recognised in vectorisable
+    // chunks, given up at the first one that differs; any other frame takes
+    // the checks atom by atom
+    const double m0 = mass[0];
+    bool uniform = m0 > 0.0;
+    for (int64_t i0 = 0; uniform && i0 < n; i0 += 1024) {
+        const int64_t i1 = std::min<int64_t>(n, i0 + 1024);
+        int differ = 0;
+        for (int64_t i = i0; i < i1; ++i)
+            differ |= mass[i] != m0;
+        if (type)
+            for (int64_t i = i0; i < i1; ++i)
+                differ |= type[i];
+        uniform = differ == 0;
+    }
+    if (uniform) {
+        seen[0] = true;
+        mt[0] = mass[0];
+    } else {
+        for (int64_t i = 0; i < n; ++i) {
+            const int t = type ? type[i] : 0;
+            if (t < 0 || t >= kMaxTypes)
+                throw Error(ATVH_E_ARG, "atvh_frame_upload: type out of range [0,16)");
+            if (!(mass[i] > 0.0))
+                throw Error(ATVH_E_ARG, "atvh_frame_upload: mass must be positive");
+            if (!seen[t]) {
+                seen[t] = true;
+                mt[t] = mass[i];
+            } else if (mt[t] != mass[i]) {
+                throw Error(ATVH_E_ARG, "atvh_frame_upload: atoms of one type must share one mass");
+            }
+            if (t + 1 > ntypes)
+                ntypes = t + 1;
         }
-        if (t + 1 > ntypes)
-            ntypes = t + 1;
     }
     for (int t = 0; t < ntypes; ++t)
         s->mass_t[t] = seen[t] ? mt[t] : 1.0;
     s->ntypes = ntypes;
     hipStream_t st = c->stream;
-    auto up = [&](double* d, const double* h) {
-        if (h)
-            ATVH_HIP(hipMemcpyAsync(d, h, n * sizeof(double), hipMemcpyHostToDevice, st));
+    // the state columns x .. q are the first ten of the frame's allocation
+    const double* cols[] = {x, y, z, vx, vy, vz, fx, fy, fz, charge};
+    constexpr int kUp = sizeof(cols) / sizeof(cols[0]);
+    const size_t nb = size_t(n) * sizeof(double), cb = size_t(s->col) * sizeof(double);
+    const size_t staged = kUp * cb + size_t(n) * sizeof(int);
+    if (staged <= kStageMax) {
+        char* pin = static_cast<char*>(ctx_pin(c, staged));
+        for (int k = 0; k < kUp; ++k) {
+            if (cols[k])
+                std::memcpy(pin + k * cb, cols[k], nb);
+            else
+                std::memset(pin + k * cb, 0, nb);
+        }
+        char* tp = pin + kUp * cb;
+        if (type)
+            std::memcpy(tp, type, size_t(n) * sizeof(int));
         else
-            ATVH_HIP(hipMemsetAsync(d, 0, n * sizeof(double), st));
-    };
-    up(s->x, x);
-    up(s->y, y);
-    up(s->z, z);
-    up(s->vx, vx);
-    up(s->vy, vy);
-    up(s->vz, vz);
-    up(s->fx, fx);
-    up(s->fy, fy);
-    up(s->fz, fz);
-    up(s->q, charge);
+            std::memset(tp, 0, size_t(n) * sizeof(int));
+        ATVH_HIP(hipMemcpyAsync(s->slab, pin, kUp * cb, hipMemcpyHostToDevice, st));
+        ATVH_HIP(hipMemcpyAsync(s->type, tp, size_t(n) * sizeof(int), hipMemcpyHostToDevice, st));
+    } else {
+        for (int k = 0; k < kUp; ++k) {
+            double* d = s->slab + k * s->col;
+            if (cols[k])
+                ATVH_HIP(hipMemcpyAsync(d, cols[k], nb, hipMemcpyHostToDevice, st));
+            else
+                ATVH_HIP(hipMemsetAsync(d, 0, nb, st));
+        }
+        if (type)
+            ATVH_HIP(hipMemcpyAsync(s->type, type, n * sizeof(int), hipMemcpyHostToDevice, st));
+        else
+            ATVH_HIP(hipMemsetAsync(s->type, 0, n * sizeof(int), st));
+    }
     s->has_charge = charge != nullptr;
     // charge sums in ascending atom order (KSpacePME self / net-charge terms,
     // pme.cpp:222-226) and the bound of any spread grid point
@@ -422,19 +529,9 @@ int atvh_frame_upload(atvh_system* s, const double* x, const double* y, const do
             s->q_abs += std::fabs(charge[i]);
             s->q_max = std::max(s->q_max, std::fabs(charge[i]));
         }
-    if (type)
-        ATVH_HIP(hipMemcpyAsync(s->type, type, n * sizeof(int), hipMemcpyHostToDevice, st));
-    else
-        ATVH_HIP(hipMemsetAsync(s->type, 0, n * sizeof(int), st));
-    k_iota<<<grid_capped(n), kBlock, 0, st>>>(n, s->tag);
-    ATVH_HIP(hipGetLastError());
     // a fresh frame: no pending thermostat scale; list must be rebuilt
-    ATVH_HIP(hipStreamSynchronize(st));
-    DevCtl h{};
-    ATVH_HIP(hipMemcpy(&h, s->ctl, sizeof(h), hipMemcpyDeviceToHost));
-    h.nh_scale = 1.0;
-    h.always = 1;
-    ATVH_HIP(hipMemcpyAsync(s->ctl, &h, sizeof(h), hipMemcpyHostToDevice, st));
+    k_frame_reset<<<grid_capped(n), kBlock, 0, st>>>(n, s->tag, s->ctl);
+    ATVH_HIP(hipGetLastError());
     s->nl_built = false;
     ATVH_HIP(hipStreamSynchronize(st));
     return ATVH_OK;
@@ -450,24 +547,22 @@ int atvh_frame_download(atvh_system* s, double* x, double* y, double* z, double*
     ATVH_HIP(hipSetDevice(c->device));
     const int64_t n = s->n;
     hipStream_t st = c->stream;
-    auto fetch3 = [&](const double* a, const double* b, const double* cc, double* ha, double* hb,
-                      double* hc, int mode) {
-        if (!ha && !hb && !hc)
-            return;
-        k_gather_out<<<grid_capped(n), kBlock, 0, st>>>(n, s->tag, a, b, cc, s->ax, s->ay, s->az,
-                                                        s->ctl, mode, s->box[0], s->box[1], s->box[2]);
-        ATVH_HIP(hipGetLastError());
-        if (ha)
-            ATVH_HIP(hipMemcpyAsync(ha, s->ax, n * sizeof(double), hipMemcpyDeviceToHost, st));
-        if (hb)
-            ATVH_HIP(hipMemcpyAsync(hb, s->ay, n * sizeof(double), hipMemcpyDeviceToHost, st));
-        if (hc)
-            ATVH_HIP(hipMemcpyAsync(hc, s->az, n * sizeof(double), hipMemcpyDeviceToHost, st));
-        ATVH_HIP(hipStreamSynchronize(st));
-    };
-    fetch3(s->x, s->y, s->z, x, y, z, 2);
-    fetch3(s->vx, s->vy, s->vz, vx, vy, vz, 1);
-    fetch3(s->fx, s->fy, s->fz, fx, fy, fz, 0);
+    double* host[] = {x, y, z, vx, vy, vz, fx, fy, fz};
+    int groups = 0;
+    for (int k = 0; k < 9; ++k)
+        groups |= host[k] ? 1 << (k / 3) : 0;
+    if (!groups)
+        return ATVH_OK;
+    // the state columns, then their frame-order copies in the permutation
+    // scratch (the same order there): one launch, one copy
+    k_gather_out<<<grid_capped(n), kBlock, 0, st>>>(n, s->col, s->tag, s->x, s->ax, s->ctl, groups, s->box[0],
+                                                    s->box[1], s->box[2]);
+    ATVH_HIP(hipGetLastError());
+    std::vector<HostPiece> pieces;
+    for (int k = 0; k < 9; ++k)
+        if (host[k])
+            pieces.push_back(HostPiece{host[k], s->ax + k * s->col, size_t(n) * sizeof(double)});
+    fetch_pieces(c, pieces);
     return ATVH_OK;
     API_CATCH(c)
 }
@@ -478,8 +573,7 @@ int atvh_energy(atvh_system* s, double* pe, double* virial6, double* ke) {
     atvh_ctx* c = s->ctx;
     API_TRY
     DevCtl h{};
-    ATVH_HIP(hipStreamSynchronize(c->stream));
-    ATVH_HIP(hipMemcpy(&h, s->ctl, sizeof(h), hipMemcpyDeviceToHost));
+    read_ctl(s, h);
     if (pe)
         *pe = h.pe;
     if (virial6)
@@ -496,9 +590,8 @@ int atvh_thermostat_state(atvh_system* s, double* xi_out, const double* xi_in) {
         return ATVH_E_ARG;
     atvh_ctx* c = s->ctx;
     API_TRY
-    ATVH_HIP(hipStreamSynchronize(c->stream));
     DevCtl h{};
-    ATVH_HIP(hipMemcpy(&h, s->ctl, sizeof(h), hipMemcpyDeviceToHost));
+    read_ctl(s, h);
     if (xi_out)
         *xi_out = h.xi;
     if (xi_in) {

@@ -543,10 +543,9 @@ void md_enqueue_steps(atvh_system* s, int first, int nsteps, int precision, int 
 // resumes at that force phase, so the trajectory equals an uninterrupted
 // run with a larger capacity.
 void md_recover_and_finish(atvh_system* s, int nsteps, int precision, int energy_every) {
-    hipStream_t st = s->ctx->stream;
     for (int attempt = 0;; ++attempt) {
         DevCtl h{};
-        ATVH_HIP(hipMemcpy(&h, s->ctl, sizeof(h), hipMemcpyDeviceToHost));
+        read_ctl(s, h);
         if (!(h.overflow || h.halo_overflow))
             return;
         if (attempt >= 8 || h.steps_done >= nsteps) {
@@ -555,7 +554,6 @@ void md_recover_and_finish(atvh_system* s, int nsteps, int precision, int energy
         }
         nl_build(s, true);
         md_enqueue_steps(s, h.steps_done, nsteps, precision, energy_every, true, thermo_rec(s));
-        ATVH_HIP(hipStreamSynchronize(st));
     }
 }
 
@@ -662,9 +660,8 @@ int atvh_integrator_configure(atvh_system* s, double dt, int thermostat, double 
     s->ndof = ndof > 0 ? ndof : 3 * s->n - 3;
     npt_free(s); // VelocityVerlet (+ NoseHoover) replaces a NoseHooverNPT
     ATVH_HIP(hipSetDevice(c->device));
-    ATVH_HIP(hipStreamSynchronize(c->stream));
     DevCtl h{};
-    ATVH_HIP(hipMemcpy(&h, s->ctl, sizeof(h), hipMemcpyDeviceToHost));
+    read_ctl(s, h);
     // NoseHoover::build: Q = Ndof kB T tau^2
     h.nh_Q = static_cast<double>(s->ndof) * kB_ev_per_k * T_target * tau_T * tau_T;
     h.nh_ndof_kT = static_cast<double>(s->ndof) * kB_ev_per_k * T_target;
@@ -738,14 +735,12 @@ int atvh_md_run(atvh_system* s, int nsteps, int precision, int energy_every) {
     }
     if (nsteps > 0) {
         // NaN marks steps without an energy request; layout [pe | ke], stride thermo_cap
-        std::vector<double> nanv(size_t(2) * s->thermo_cap, std::nan(""));
-        ATVH_HIP(hipMemcpyAsync(s->d_thermo, nanv.data(), nanv.size() * sizeof(double),
-                                hipMemcpyHostToDevice, st));
-        ATVH_HIP(hipStreamSynchronize(st));
+        k_fill_records<<<(s->thermo_cap + kBlock - 1) / kBlock, kBlock, 0, st>>>(s->d_thermo, s->thermo_cap,
+                                                                                 s->thermo_cap);
+        ATVH_HIP(hipGetLastError());
     }
     k_run_reset<<<1, 64, 0, st>>>(s->ctl);
     md_enqueue_steps(s, 0, nsteps, precision, energy_every, false, thermo_rec(s));
-    ATVH_HIP(hipStreamSynchronize(st));
     md_recover_and_finish(s, nsteps, precision, energy_every);
     return ATVH_OK;
     API_CATCH(c)
@@ -790,9 +785,8 @@ int atvh_md_run_noalloc(atvh_system* s, int nsteps, int precision, int energy_ev
     s->thermo_n = 0; // the system's own record no longer describes the last run
     k_run_reset<<<1, 64, 0, st>>>(s->ctl);
     md_enqueue_steps(s, 0, nsteps, precision, energy_every, false, ThermoRec{rec, rec + kNoAllocSteps});
-    ATVH_HIP(hipStreamSynchronize(st));
     DevCtl h{};
-    ATVH_HIP(hipMemcpy(&h, s->ctl, sizeof(h), hipMemcpyDeviceToHost));
+    read_ctl(s, h);
     if (h.overflow || h.halo_overflow) {
         // regrowing the list would allocate: the system stays halted at the
         // step whose rebuild overflowed and the caller re-uploads its frame
@@ -830,9 +824,8 @@ int atvh_stress(atvh_system* s, double* kinetic6, double* virial6, double* press
     atvh_ctx* c = s->ctx;
     API_TRY
     ATVH_HIP(hipSetDevice(c->device));
-    ATVH_HIP(hipStreamSynchronize(c->stream));
     DevCtl h{};
-    ATVH_HIP(hipMemcpy(&h, s->ctl, sizeof(h), hipMemcpyDeviceToHost));
+    read_ctl(s, h);
     if (kinetic6)
         for (int k = 0; k < 6; ++k)
             kinetic6[k] = h.stress_kin[k];
@@ -857,14 +850,16 @@ int atvh_md_thermo(atvh_system* s, double* pe, double* ke, int nsteps) {
     API_TRY
     if (nsteps > s->thermo_n)
         throw Error(ATVH_E_ARG, "atvh_md_thermo: more steps requested than recorded");
-    ATVH_HIP(hipStreamSynchronize(c->stream));
-    if (nsteps <= 0)
+    if (nsteps <= 0) {
+        ATVH_HIP(hipStreamSynchronize(c->stream));
         return ATVH_OK;
+    }
+    std::vector<HostPiece> pieces;
     if (pe)
-        ATVH_HIP(hipMemcpy(pe, s->d_thermo, nsteps * sizeof(double), hipMemcpyDeviceToHost));
+        pieces.push_back(HostPiece{pe, s->d_thermo, nsteps * sizeof(double)});
     if (ke)
-        ATVH_HIP(hipMemcpy(ke, s->d_thermo + s->thermo_cap, nsteps * sizeof(double),
-                           hipMemcpyDeviceToHost));
+        pieces.push_back(HostPiece{ke, s->d_thermo + s->thermo_cap, nsteps * sizeof(double)});
+    fetch_pieces(c, pieces);
     return ATVH_OK;
     API_CATCH(c)
 }

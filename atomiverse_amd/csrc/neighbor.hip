@@ -1112,6 +1112,46 @@ __global__ void k_nl_stats_reset(DevCtl* ctl) {
     }
 }
 
+constexpr int kFillThreads = 1024;
+
+__global__ __launch_bounds__(kFillThreads) void k_nl_brick_fill(int nbricks, const int* __restrict__ halo_n,
+                                                                const int2* __restrict__ range, DevCtl* ctl) {
+    __shared__ int sh[2][kFillThreads / 64];
+    int mh = 0, ma = 0;
+    for (int b = threadIdx.x; b < nbricks; b += kFillThreads) {
+        mh = max(mh, halo_n[b]);
+        ma = max(ma, range[b].y);
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        mh = max(mh, __shfl_down(mh, off, 64));
+        ma = max(ma, __shfl_down(ma, off, 64));
+    }
+    if ((threadIdx.x & 63) == 0) {
+        sh[0][threadIdx.x >> 6] = mh;
+        sh[1][threadIdx.x >> 6] = ma;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < kFillThreads / 64; ++w) {
+            mh = max(mh, sh[0][w]);
+            ma = max(ma, sh[1][w]);
+        }
+        ctl->fill_halo = mh;
+        ctl->fill_atoms = ma;
+    }
+}
+
+// A list build that fits: the cadence counters start over.
+__global__ void k_nl_built(DevCtl* ctl, int keep_counts) {
+    if (threadIdx.x != 0 || blockIdx.x != 0)
+        return;
+    ctl->ago = 0;
+    if (!keep_counts)
+        ctl->nrebuilds = 1;
+    ctl->disp_flag = 0;
+    ctl->rebuild = 0;
+}
+
 __global__ void k_nl_export(int64_t n, const int* __restrict__ tag, const int* __restrict__ numneigh,
                             const int* __restrict__ nbr, int64_t npad,
                             const long long* __restrict__ offs, long long* __restrict__ out) {
@@ -1358,15 +1398,35 @@ void nl_setup_grid(atvh_system* s) {
     s->ncols = static_cast<int>(cols.size() / 4);
     if (s->ncols > kMaxCols)
         throw Error(ATVH_E_ARG, "stencil has more columns than the list build supports");
+    // capacity: 1.5x the mean full-list count at this density, plus margin
+    const double vol = s->box[0] * s->box[1] * s->box[2];
+    const double mean = double(s->n) / vol * 4.18879020478639 * cutoff_skin * cutoff_skin * cutoff_skin;
+    int cap = static_cast<int>(std::ceil(1.5 * mean + 32));
+    cap = (cap + 7) / 8 * 8;
+    if (cap > s->n)
+        cap = static_cast<int>(std::max<int64_t>(8, (s->n + 7) / 8 * 8));
+    // A box that moved (NoseHooverNPT, a rebuild every few steps) mostly keeps
+    // its cell counts: the tables depend on those, the brick shape and the
+    // stencil alone, so they and the buffers stay (25 allocations and their
+    // synchronising frees otherwise)
+    std::vector<int> sig(st);
+    sig.insert(sig.end(), cols.begin(), cols.end());
+    s->brick_mode = s->use_half;
+    if (s->brick_mode)
+        choose_bricks(s, s->brick_pick_min);
+    sig.insert(sig.end(), {s->nc[0], s->nc[1], s->nc[2], s->reach[0], s->reach[1], s->reach[2],
+                           s->brick_mode ? s->brick_pick : -1});
+    if (s->cell_rank && sig == s->nl_sig) {
+        if (s->cap < cap)
+            nl_realloc_capacity(s, cap);
+        return;
+    }
     nl_free(s);
     dev_alloc(&s->d_cols, cols.size());
     ATVH_HIP(hipMemcpy(s->d_cols, cols.data(), cols.size() * sizeof(int), hipMemcpyHostToDevice));
     // brick layout when the half-stencil arithmetic applies, else one brick
     // per cell and the global-slot fallback list
-    s->brick_mode = s->use_half;
-    if (s->brick_mode) {
-        choose_bricks(s, s->brick_pick_min);
-    } else {
+    if (!s->brick_mode) {
         for (int a = 0; a < 3; ++a) {
             s->bdim[a] = 1;
             s->nb[a] = s->nc[a];
@@ -1415,17 +1475,12 @@ void nl_setup_grid(atvh_system* s) {
         dev_alloc(&s->halo_n, s->nbricks);
         dev_alloc(&s->brick_range, s->nbricks);
     }
-    // capacity: 1.5x the mean full-list count at this density, plus margin
-    const double vol = s->box[0] * s->box[1] * s->box[2];
-    const double mean = double(s->n) / vol * 4.18879020478639 * cutoff_skin * cutoff_skin * cutoff_skin;
-    int cap = static_cast<int>(std::ceil(1.5 * mean + 32));
-    cap = (cap + 7) / 8 * 8;
-    if (cap > s->n)
-        cap = static_cast<int>(std::max<int64_t>(8, (s->n + 7) / 8 * 8));
     nl_realloc_capacity(s, cap);
+    s->nl_sig = std::move(sig);
 }
 
 void nl_free(atvh_system* s) {
+    s->nl_sig.clear();
     dev_free(s->d_stencil);
     dev_free(s->halo_cells);
     dev_free(s->d_cols);
@@ -1654,6 +1709,10 @@ void nl_batch_build(atvh_batch* b) {
     std::vector<int> nb;
     for (int k = 0; k < kNlStages; ++k)
         nb.insert(nb.end(), g[k].begin(), g[k].end());
+    if (b->nl_nb && nb == b->nl_blocks)
+        return;
+    b->nl_blocks = nb;
+    b->stages_changed = true;
     dev_free(b->nl_nb);
     dev_free(b->nl_act);
     dev_free(b->nl_flags);
@@ -1740,19 +1799,19 @@ void nl_check_ctl(const DevCtl& h) {
         throw Error(ATVH_E_CAPACITY, "neighbor capacity exceeded during a rebuild");
 }
 
-// Fullest halo and brick of the last build (per-brick counts read back; a
-// list build only).
+// Fullest halo and brick of the current list, left in the control block (one
+// block over the per-brick counts; a list build and brick queries only).
+static void enqueue_brick_fill(atvh_system* s) {
+    k_nl_brick_fill<<<1, kFillThreads, 0, s->ctx->stream>>>(s->nbricks, s->halo_n, s->brick_range, s->ctl);
+    ATVH_HIP(hipGetLastError());
+}
+
 static void brick_fill(atvh_system* s, int& max_halo, int& max_atoms) {
-    std::vector<int> hn(s->nbricks);
-    std::vector<int2> br(s->nbricks);
-    ATVH_HIP(hipMemcpy(hn.data(), s->halo_n, hn.size() * sizeof(int), hipMemcpyDeviceToHost));
-    ATVH_HIP(hipMemcpy(br.data(), s->brick_range, br.size() * sizeof(int2), hipMemcpyDeviceToHost));
-    max_halo = 0;
-    max_atoms = 0;
-    for (int b = 0; b < s->nbricks; ++b) {
-        max_halo = std::max(max_halo, hn[b]);
-        max_atoms = std::max(max_atoms, br[b].y);
-    }
+    enqueue_brick_fill(s);
+    DevCtl h{};
+    read_ctl(s, h);
+    max_halo = h.fill_halo;
+    max_atoms = h.fill_atoms;
 }
 
 void nl_build(atvh_system* s, bool keep_counts) {
@@ -1761,27 +1820,21 @@ void nl_build(atvh_system* s, bool keep_counts) {
         k_nl_stats_reset<<<1, 64, 0, c->stream>>>(s->ctl);
         // the initial build also orders the frame's forces (first kick uses them)
         nl_enqueue_rebuild(s, &s->ctl->always, true);
-        ATVH_HIP(hipStreamSynchronize(c->stream));
+        if (s->brick_mode)
+            enqueue_brick_fill(s);
         DevCtl h{};
-        ATVH_HIP(hipMemcpy(&h, s->ctl, sizeof(h), hipMemcpyDeviceToHost));
+        read_ctl(s, h);
         // a brick shape whose fullest halo or brick (measured on these
         // positions) leaves less than a sixteenth of the LDS rows or of the
         // brick's atom slots free is given up for the next smaller one:
         // denser-than-uniform inputs keep some headroom for the rebuilds of
         // the run
         bool tight = false;
-        if (s->brick_mode && s->brick_pick < kLastBrickCand && h.halo_overflow == 0) {
-            int max_halo = 0, max_atoms = 0;
-            brick_fill(s, max_halo, max_atoms);
-            tight = max_halo > kHaloFillMax || max_atoms > brick_atom_limit(s) * 15 / 16;
-        }
+        if (s->brick_mode && s->brick_pick < kLastBrickCand && h.halo_overflow == 0)
+            tight = h.fill_halo > kHaloFillMax || h.fill_atoms > brick_atom_limit(s) * 15 / 16;
         if (h.overflow == 0 && h.halo_overflow == 0 && !tight) {
-            h.ago = 0;
-            if (!keep_counts)
-                h.nrebuilds = 1;
-            h.disp_flag = 0;
-            h.rebuild = 0;
-            ATVH_HIP(hipMemcpy(s->ctl, &h, sizeof(h), hipMemcpyHostToDevice));
+            k_nl_built<<<1, 64, 0, c->stream>>>(s->ctl, keep_counts ? 1 : 0);
+            ATVH_HIP(hipGetLastError());
             s->nl_built = true;
             for (int d = 0; d < 3; ++d)
                 s->nl_box[d] = s->box[d];
@@ -2046,9 +2099,8 @@ int atvh_nlist_decide_and_rebuild(atvh_system* s) {
     // the overflow probe is read back here, as the reference's list rebuild
     // reads its pair count (src/cuda/neighbor/neighbor_list.cu:544-553): an
     // overflowing rebuild is redone at once with a grown capacity
-    ATVH_HIP(hipStreamSynchronize(c->stream));
     DevCtl h{};
-    ATVH_HIP(hipMemcpy(&h, s->ctl, sizeof(h), hipMemcpyDeviceToHost));
+    read_ctl(s, h);
     if (h.overflow || h.halo_overflow)
         nl_build(s, true);
     return ATVH_OK;
@@ -2061,9 +2113,8 @@ int atvh_nlist_stats(atvh_system* s, int64_t* nrebuilds, int64_t* npairs_half, i
         return ATVH_E_ARG;
     atvh_ctx* c = s->ctx;
     API_TRY
-    ATVH_HIP(hipStreamSynchronize(c->stream));
     DevCtl h{};
-    ATVH_HIP(hipMemcpy(&h, s->ctl, sizeof(h), hipMemcpyDeviceToHost));
+    read_ctl(s, h);
     if (nrebuilds)
         *nrebuilds = h.nrebuilds;
     if (npairs_half)
@@ -2089,8 +2140,7 @@ int atvh_nlist_export_pairs(atvh_system* s, int64_t* pairs, int64_t cap, int64_t
     const int64_t n = s->n;
     {
         DevCtl hc{};
-        ATVH_HIP(hipStreamSynchronize(st));
-        ATVH_HIP(hipMemcpy(&hc, s->ctl, sizeof(hc), hipMemcpyDeviceToHost));
+        read_ctl(s, hc);
         nl_check_ctl(hc);
     }
     long long* d_cnt = nullptr;

@@ -282,11 +282,6 @@ NptArgs npt_args(atvh_system* s) {
     return a;
 }
 
-void read_ctl(atvh_system* s, DevCtl& h) {
-    ATVH_HIP(hipStreamSynchronize(s->ctx->stream));
-    ATVH_HIP(hipMemcpy(&h, s->ctl, sizeof(h), hipMemcpyDeviceToHost));
-}
-
 void reduce(atvh_system* s, const NptArgs& a, int cols) {
     k_npt_sum<<<1, kBlock, 0, s->ctx->stream>>>(a.partials, a.nb, cols, s->ctl);
     ATVH_HIP(hipGetLastError());

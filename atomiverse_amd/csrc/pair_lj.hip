@@ -773,8 +773,16 @@ void pair_batch_build(atvh_batch* b) {
     if (typed_any && !typed_all)
         throw Error(ATVH_E_ARG, "batch: PairLJCut members must all be single-type or all per-type");
     b->typed = typed_any;
-    if (!args.empty())
+    if (!args.empty()) {
         batch_stage(b, "pair", args, blocks);
+    } else if (const auto it = b->stages.find("pair"); it != b->stages.end()) {
+        // every member's force call is its own now
+        dev_free(it->second.args);
+        dev_free(it->second.base);
+        dev_free(it->second.owner);
+        b->stages.erase(it);
+        b->stages_changed = true;
+    }
 }
 
 template <class Op>
