@@ -478,14 +478,15 @@ template <bool EF, bool VF, bool MIXED>
 __global__ __launch_bounds__(kBlock) void k_ljc_global(LjcArgs a) {
     double acc[7] = {0, 0, 0, 0, 0, 0, 0};
     const int ntypes = a.ntypes, nbin1 = a.nbin - 1;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < a.n;
-         i += (int64_t)gridDim.x * blockDim.x) {
+    const int sub = threadIdx.x % kSmallLanes;
+    for (int64_t i = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) / kSmallLanes; i < a.n;
+         i += (int64_t)gridDim.x * blockDim.x / kSmallLanes) {
         const double xi = a.x[i], yi = a.y[i], zi = a.z[i];
         const double qi_scale = coulomb * a.q[i];
         const int ti = a.type[i];
         const int nn = a.numneigh[i];
         double fxi = 0.0, fyi = 0.0, fzi = 0.0;
-        for (int k = 0; k < nn; ++k) {
+        for (int k = sub; k < nn; k += kSmallLanes) {
             const int j = a.nbr[(int64_t)k * a.npad + i];
             double dx = xi - a.x[j];
             double dy = yi - a.y[j];
@@ -539,9 +540,14 @@ __global__ __launch_bounds__(kBlock) void k_ljc_global(LjcArgs a) {
                 acc[6] += dy * fzp;
             }
         }
-        a.fx[i] = fxi;
-        a.fy[i] = fyi;
-        a.fz[i] = fzi;
+        small_lane_sum(fxi);
+        small_lane_sum(fyi);
+        small_lane_sum(fzi);
+        if (sub == 0) {
+            a.fx[i] = fxi;
+            a.fy[i] = fyi;
+            a.fz[i] = fzi;
+        }
     }
     if (EF || VF) {
 #pragma unroll

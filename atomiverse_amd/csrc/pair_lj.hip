@@ -53,14 +53,15 @@ struct LJArgs {
 template <bool EF, bool VF, bool TYPED>
 __global__ __launch_bounds__(kBlock) void k_lj_fp64(int64_t n, LJArgs a) {
     double acc[7] = {0, 0, 0, 0, 0, 0, 0};
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x) {
+    const int sub = threadIdx.x % kSmallLanes;
+    for (int64_t i = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) / kSmallLanes; i < n;
+         i += (int64_t)gridDim.x * blockDim.x / kSmallLanes) {
         const double xi = a.x[i], yi = a.y[i], zi = a.z[i];
         const int ti = TYPED ? a.type[i] : 0;
         const int nn = a.numneigh[i];
         double fxi = 0.0, fyi = 0.0, fzi = 0.0;
         const int* __restrict__ col = a.nbr + i;
-        for (int k = 0; k < nn; ++k) {
+        for (int k = sub; k < nn; k += kSmallLanes) {
             const int j = col[(int64_t)k * a.npad];
             double dx = xi - a.x[j];
             double dy = yi - a.y[j];
@@ -97,9 +98,14 @@ __global__ __launch_bounds__(kBlock) void k_lj_fp64(int64_t n, LJArgs a) {
                 }
             }
         }
-        a.fx[i] = fxi;
-        a.fy[i] = fyi;
-        a.fz[i] = fzi;
+        small_lane_sum(fxi);
+        small_lane_sum(fyi);
+        small_lane_sum(fzi);
+        if (sub == 0) {
+            a.fx[i] = fxi;
+            a.fy[i] = fyi;
+            a.fz[i] = fzi;
+        }
     }
     if (EF || VF) {
 #pragma unroll
@@ -114,14 +120,15 @@ __global__ __launch_bounds__(kBlock) void k_lj_mixed(int64_t n, LJArgs a) {
     double acc[7] = {0, 0, 0, 0, 0, 0, 0};
     const float eps24s = static_cast<float>(a.eps24), eps4s = static_cast<float>(a.eps4);
     const float sig6s = static_cast<float>(a.sig6), shifts = static_cast<float>(a.vshift);
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x) {
+    const int sub = threadIdx.x % kSmallLanes;
+    for (int64_t i = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) / kSmallLanes; i < n;
+         i += (int64_t)gridDim.x * blockDim.x / kSmallLanes) {
         const double xi = a.x[i], yi = a.y[i], zi = a.z[i];
         const int ti = TYPED ? a.type[i] : 0;
         const int nn = a.numneigh[i];
         float fxi = 0.f, fyi = 0.f, fzi = 0.f;
         const int* __restrict__ col = a.nbr + i;
-        for (int k = 0; k < nn; ++k) {
+        for (int k = sub; k < nn; k += kSmallLanes) {
             const int j = col[(int64_t)k * a.npad];
             double dxd = xi - a.x[j];
             double dyd = yi - a.y[j];
@@ -162,9 +169,14 @@ __global__ __launch_bounds__(kBlock) void k_lj_mixed(int64_t n, LJArgs a) {
                 }
             }
         }
-        a.fx[i] = static_cast<double>(fxi);
-        a.fy[i] = static_cast<double>(fyi);
-        a.fz[i] = static_cast<double>(fzi);
+        small_lane_sum(fxi);
+        small_lane_sum(fyi);
+        small_lane_sum(fzi);
+        if (sub == 0) {
+            a.fx[i] = static_cast<double>(fxi);
+            a.fy[i] = static_cast<double>(fyi);
+            a.fz[i] = static_cast<double>(fzi);
+        }
     }
     if (EF || VF) {
 #pragma unroll
@@ -609,7 +621,7 @@ static void lj_brick_dispatch(atvh_ctx* c, bool ef, bool vf, bool ty, int grid, 
 
 namespace atvh {
 
-int pair_grid(const atvh_system* s) { return s->brick_mode ? s->nbricks : grid_capped(s->n); }
+int pair_grid(const atvh_system* s) { return s->brick_mode ? s->nbricks : grid_capped(s->n * kSmallLanes); }
 
 static void lj_enqueue(atvh_system* s, int precision, bool eflag, bool vflag);
 
