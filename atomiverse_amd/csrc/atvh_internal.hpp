@@ -24,6 +24,7 @@ constexpr double coulomb = 14.399645;
 constexpr int kMaxTypes = 16;
 constexpr int kBlock = 256;       // threads per workgroup (4 wave64)
 constexpr int kMaxGrid = 8192;    // cap for grid-stride kernels that may be predicated off
+constexpr int kStepKinds = 3;     // batched steps: forces, + energies, + virials
 constexpr int kPartialStride = 8; // doubles per block partial (pe, vir[6], spare)
 
 struct Error : std::runtime_error {
@@ -243,8 +244,9 @@ struct atvh_batch {
     // LJ + Coulomb with or without PME): queued one by one inside the step
     std::vector<atvh_system*> solo;
     bool use_graph = false;
-    hipGraphExec_t graph[2] = {nullptr, nullptr}; // [energy step?]
-    int graph_prec[2] = {-1, -1};
+    // captured steps: forces only, with energies, with energies and virials
+    hipGraphExec_t graph[atvh::kStepKinds] = {nullptr, nullptr, nullptr};
+    int graph_prec[atvh::kStepKinds] = {-1, -1, -1};
     int thermo_cap = 0;
     int* d_slot_member = nullptr; // replica exchange: member holding ladder slot k
     int* d_accept = nullptr;      // accepted exchanges of the last round
@@ -347,7 +349,7 @@ void pair_free(atvh_system* s);
 
 // coul_pme.hip
 void ljc_enqueue(atvh_system* s, int precision, bool eflag, bool vflag);
-void pme_enqueue(atvh_system* s, int precision, bool ev);
+void pme_enqueue(atvh_system* s, int precision, int ev);
 int pme_partial_blocks(const atvh_system* s);
 // true when the PME buffers and transform plans of this precision exist (or
 // no PME is configured), so a step allocates nothing
@@ -372,7 +374,7 @@ void integ_batch_launch(atvh_batch* b, const char* stage);
 void nl_batch_build(atvh_batch* b);
 void nl_batch_launch_rebuild(atvh_batch* b);
 void pair_batch_build(atvh_batch* b);
-void pair_batch_launch(atvh_batch* b, int precision, bool ef);
+void pair_batch_launch(atvh_batch* b, int precision, bool ef, bool vf);
 
 // device bytes held per component (atvh_system_memory)
 int64_t nl_device_bytes(const atvh_system* s);

@@ -97,7 +97,7 @@ __global__ void k_batch_exchange(DevCtl** ctls, int* slot_member, int nslots, in
 }
 
 void free_graphs(atvh_batch* b) {
-    for (int k = 0; k < 2; ++k) {
+    for (int k = 0; k < kStepKinds; ++k) {
         if (b->graph[k])
             (void)hipGraphExecDestroy(b->graph[k]);
         b->graph[k] = nullptr;
@@ -109,7 +109,7 @@ void free_graphs(atvh_batch* b) {
 // captured) each launch family is bracketed by events of its own, named
 // apart from the single-system families (a charged member's own force call
 // inside the pair family times itself as "pair").
-void enqueue_step(atvh_batch* b, int precision, bool ef) {
+void enqueue_step(atvh_batch* b, int precision, bool ef, bool vf) {
     atvh_ctx* c = b->ctx;
     {
         ScopedTimer tm(c, "batch_integrate");
@@ -122,7 +122,7 @@ void enqueue_step(atvh_batch* b, int precision, bool ef) {
     }
     {
         ScopedTimer tm(c, "batch_pair");
-        pair_batch_launch(b, precision, ef);
+        pair_batch_launch(b, precision, ef, vf);
     }
     if (ef) {
         ScopedTimer tm(c, "batch_energy");
@@ -301,17 +301,20 @@ int atvh_batch_run(atvh_batch* b, int nsteps, int precision, int energy_every) {
     for (atvh_system* s : b->solo)
         kspace = kspace || s->pme != nullptr;
     for (int step = 0; step < nsteps; ++step) {
-        const bool ef = (step == nsteps - 1) || (energy_every > 0 && (step % energy_every) == 0);
+        // the virial is not recorded per step: only the last one can be read
+        const bool vf = step == nsteps - 1;
+        const bool ef = vf || (energy_every > 0 && (step % energy_every) == 0);
+        const int kind = vf ? 2 : (ef ? 1 : 0);
         if (b->use_graph && !timing && !kspace) {
-            hipGraphExec_t& ge = b->graph[ef ? 1 : 0];
-            if (!ge || b->graph_prec[ef ? 1 : 0] != precision) {
+            hipGraphExec_t& ge = b->graph[kind];
+            if (!ge || b->graph_prec[kind] != precision) {
                 if (ge)
                     ATVH_HIP(hipGraphExecDestroy(ge));
                 ge = nullptr;
                 hipGraph_t g = nullptr;
                 ATVH_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
                 try {
-                    enqueue_step(b, precision, ef);
+                    enqueue_step(b, precision, ef, vf);
                 } catch (...) {
                     (void)hipStreamEndCapture(st, &g);
                     if (g)
@@ -322,12 +325,12 @@ int atvh_batch_run(atvh_batch* b, int nsteps, int precision, int energy_every) {
                 const hipError_t e = hipGraphInstantiate(&ge, g, nullptr, nullptr, 0);
                 (void)hipGraphDestroy(g);
                 ATVH_HIP(e);
-                b->graph_prec[ef ? 1 : 0] = precision;
+                b->graph_prec[kind] = precision;
             }
             ATVH_HIP(hipGraphLaunch(ge, st));
         } else {
             ScopedTimer tm(c, "batch_step");
-            enqueue_step(b, precision, ef);
+            enqueue_step(b, precision, ef, vf);
         }
     }
     // a member whose rebuild overflowed its list capacity or a brick halo

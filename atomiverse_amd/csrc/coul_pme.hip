@@ -895,7 +895,8 @@ __global__ __launch_bounds__(kBlock) void k_pme_unfix(int64_t ntot, unsigned lon
 // m_a m_b of the partner changes sign unless one of the two indices is the
 // Nyquist plane of its axis (h = K/2 maps to itself), so it is folded in as
 // m_a m_b (1 + s_a s_b) with s = -1, or +1 on a Nyquist plane (s_z = -1).
-template <class T2, bool EV>
+// EV: 0 none, 1 energy, 2 energy and virial.
+template <class T2, int EV>
 __global__ __launch_bounds__(kBlock) void k_pme_influence(PmeArgs a, T2* __restrict__ cplx) {
     double acc[7] = {0, 0, 0, 0, 0, 0, 0};
     const int64_t nmodes = (int64_t)a.K0 * a.K1 * a.Kh;
@@ -905,32 +906,33 @@ __global__ __launch_bounds__(kBlock) void k_pme_influence(PmeArgs a, T2* __restr
         T2 c = cplx[idx];
         if (EV && h != 0.0) {
             const int m2 = static_cast<int>(idx % a.Kh);
-            const int64_t r = idx / a.Kh;
-            const int m1 = static_cast<int>(r % a.K1);
-            const int m0 = static_cast<int>(r / a.K1);
-            const int h0 = (m0 <= a.K0 / 2) ? m0 : m0 - a.K0;
-            const int h1 = (m1 <= a.K1 / 2) ? m1 : m1 - a.K1;
-            const int h2 = (m2 <= a.K2 / 2) ? m2 : m2 - a.K2;
-            const double mx = h0 * a.ic0, my = h1 * a.ic1, mz = h2 * a.ic2;
-            const double msq = mx * mx + my * my + mz * mz;
-            const double re = static_cast<double>(c.x), im = static_cast<double>(c.y);
-            const double q2 = re * re + im * im;
-            const double vt = -2.0 * (1.0 / msq + a.pi2_a2);
-            const double ug = h * q2;
             const bool pair = m2 != 0 && 2 * m2 != a.K2;
             const double w = pair ? 2.0 : 1.0;
-            const double sx = (2 * m0 == a.K0) ? 1.0 : -1.0;
-            const double sy = (2 * m1 == a.K1) ? 1.0 : -1.0;
-            const double oxy = pair ? 1.0 + sx * sy : 1.0;
-            const double oxz = pair ? 1.0 - sx : 1.0;
-            const double oyz = pair ? 1.0 - sy : 1.0;
+            const double re = static_cast<double>(c.x), im = static_cast<double>(c.y);
+            const double ug = h * (re * re + im * im);
             acc[0] += w * ug;
-            acc[1] += w * ug * (1.0 + vt * mx * mx);
-            acc[2] += w * ug * (1.0 + vt * my * my);
-            acc[3] += w * ug * (1.0 + vt * mz * mz);
-            acc[4] += oxy * ug * (vt * mx * my);
-            acc[5] += oxz * ug * (vt * mx * mz);
-            acc[6] += oyz * ug * (vt * my * mz);
+            if (EV == 2) {
+                const int64_t r = idx / a.Kh;
+                const int m1 = static_cast<int>(r % a.K1);
+                const int m0 = static_cast<int>(r / a.K1);
+                const int h0 = (m0 <= a.K0 / 2) ? m0 : m0 - a.K0;
+                const int h1 = (m1 <= a.K1 / 2) ? m1 : m1 - a.K1;
+                const int h2 = (m2 <= a.K2 / 2) ? m2 : m2 - a.K2;
+                const double mx = h0 * a.ic0, my = h1 * a.ic1, mz = h2 * a.ic2;
+                const double msq = mx * mx + my * my + mz * mz;
+                const double vt = -2.0 * (1.0 / msq + a.pi2_a2);
+                const double sx = (2 * m0 == a.K0) ? 1.0 : -1.0;
+                const double sy = (2 * m1 == a.K1) ? 1.0 : -1.0;
+                const double oxy = pair ? 1.0 + sx * sy : 1.0;
+                const double oxz = pair ? 1.0 - sx : 1.0;
+                const double oyz = pair ? 1.0 - sy : 1.0;
+                acc[1] += w * ug * (1.0 + vt * mx * mx);
+                acc[2] += w * ug * (1.0 + vt * my * my);
+                acc[3] += w * ug * (1.0 + vt * mz * mz);
+                acc[4] += oxy * ug * (vt * mx * my);
+                acc[5] += oxz * ug * (vt * mx * mz);
+                acc[6] += oyz * ug * (vt * my * mz);
+            }
         }
         using TS = decltype(c.x);
         c.x *= static_cast<TS>(h);
@@ -1337,7 +1339,7 @@ int ilog2(int k) {
 // potential mesh out, influence applied, energy/virial partials (ev) in
 // gm blocks.
 template <class T>
-void fft_native_enqueue(atvh_system* s, const PmeArgs& pa, bool ev, int gm, hipStream_t st) {
+void fft_native_enqueue(atvh_system* s, const PmeArgs& pa, int ev, int gm, hipStream_t st) {
     using namespace pmefft;
     PmeState* p = s->pme;
     const bool f32 = std::is_same<T, float>::value;
@@ -1375,10 +1377,12 @@ void fft_native_enqueue(atvh_system* s, const PmeArgs& pa, bool ev, int gm, hipS
 #define ATVH_FFT_B(L) k_fft_y<T, L, false><<<gb, kFftTileThreads, 0, st>>>(f)
 #define ATVH_FFT_C(L)                                                    \
     do {                                                                 \
-        if (ev)                                                          \
-            k_fft_x_influence<T, L, true><<<gm, kFftTileThreads, 0, st>>>(f); \
+        if (ev == 2)                                                     \
+            k_fft_x_influence<T, L, 2><<<gm, kFftTileThreads, 0, st>>>(f); \
+        else if (ev == 1)                                                \
+            k_fft_x_influence<T, L, 1><<<gm, kFftTileThreads, 0, st>>>(f); \
         else                                                             \
-            k_fft_x_influence<T, L, false><<<gm, kFftTileThreads, 0, st>>>(f); \
+            k_fft_x_influence<T, L, 0><<<gm, kFftTileThreads, 0, st>>>(f); \
     } while (0)
 #define ATVH_FFT_D(L) k_fft_y<T, L, true><<<gb, kFftTileThreads, 0, st>>>(f)
 #define ATVH_FFT_E(L) k_fft_c2r_z<T, L><<<ga, kFftThreads, 0, st>>>(f)
@@ -1473,7 +1477,18 @@ void pme_prepare(atvh_system* s, int precision) {
     p->nb = pme_grid_blocks(s, precision);
 }
 
-void pme_enqueue(atvh_system* s, int precision, bool ev) {
+template <class T2>
+static void launch_influence(int ev, int grid, hipStream_t st, const PmeArgs& a, T2* cplx) {
+    if (ev == 2)
+        k_pme_influence<T2, 2><<<grid, kBlock, 0, st>>>(a, cplx);
+    else if (ev == 1)
+        k_pme_influence<T2, 1><<<grid, kBlock, 0, st>>>(a, cplx);
+    else
+        k_pme_influence<T2, 0><<<grid, kBlock, 0, st>>>(a, cplx);
+}
+
+// ev: 0 forces only, 1 with the energy, 2 with the energy and the virial
+void pme_enqueue(atvh_system* s, int precision, int ev) {
     PmeState* p = s->pme;
     if (!s->has_charge)
         throw Error(ATVH_E_STATE, "KSpacePME: the frame carries no charges");
@@ -1513,10 +1528,7 @@ void pme_enqueue(atvh_system* s, int precision, bool ev) {
         k_pme_unfix<float><<<gg, kBlock, 0, st>>>(ntot, p->fix, p->real32, a.inv_fix);
         HIPFFT_CHECK(hipfftSetStream(p->f32, st));
         HIPFFT_CHECK(hipfftExecR2C(p->f32, p->real32, reinterpret_cast<hipfftComplex*>(p->cplx32)));
-        if (ev)
-            k_pme_influence<float2, true><<<gm, kBlock, 0, st>>>(a, p->cplx32);
-        else
-            k_pme_influence<float2, false><<<gm, kBlock, 0, st>>>(a, p->cplx32);
+        launch_influence<float2>(ev, gm, st, a, p->cplx32);
         HIPFFT_CHECK(hipfftSetStream(p->b32, st));
         HIPFFT_CHECK(hipfftExecC2R(p->b32, reinterpret_cast<hipfftComplex*>(p->cplx32), p->real32));
         dispatch_order<float>(p->order, false, st, a, p->real32, sr);
@@ -1525,10 +1537,7 @@ void pme_enqueue(atvh_system* s, int precision, bool ev) {
         k_pme_unfix<double><<<gg, kBlock, 0, st>>>(ntot, p->fix, p->real64, a.inv_fix);
         HIPFFT_CHECK(hipfftSetStream(p->f64, st));
         HIPFFT_CHECK(hipfftExecD2Z(p->f64, p->real64, reinterpret_cast<hipfftDoubleComplex*>(p->cplx64)));
-        if (ev)
-            k_pme_influence<double2, true><<<gm, kBlock, 0, st>>>(a, p->cplx64);
-        else
-            k_pme_influence<double2, false><<<gm, kBlock, 0, st>>>(a, p->cplx64);
+        launch_influence<double2>(ev, gm, st, a, p->cplx64);
         HIPFFT_CHECK(hipfftSetStream(p->b64, st));
         HIPFFT_CHECK(hipfftExecZ2D(p->b64, reinterpret_cast<hipfftDoubleComplex*>(p->cplx64), p->real64));
         dispatch_order<double>(p->order, false, st, a, p->real64, sr);
@@ -1828,7 +1837,7 @@ int atvh_pme_compute(atvh_system* s, int precision, int eflag, int vflag) {
     ATVH_HIP(hipSetDevice(c->device));
     k_zero3<<<grid_capped(s->n), kBlock, 0, c->stream>>>(s->n, s->fx, s->fy, s->fz);
     ATVH_HIP(hipGetLastError());
-    const bool ev = eflag || vflag;
+    const int ev = vflag ? 2 : (eflag ? 1 : 0);
     pme_enqueue(s, precision, ev);
     if (ev)
         energy_enqueue_finalize(s, nullptr, 0, false);

@@ -215,23 +215,6 @@ struct OpKinStress {
     }
 };
 
-// Fixed-order sum of nb partials (stride `stride`) over one 256-thread block.
-__device__ double block_fixed_sum(const double* p, int nb, int stride) {
-    __shared__ double sh[kBlock];
-    double t = 0.0;
-    for (int b = threadIdx.x; b < nb; b += kBlock)
-        t += p[(int64_t)b * stride];
-    sh[threadIdx.x] = t;
-    __syncthreads();
-    for (int off = kBlock / 2; off > 0; off >>= 1) {
-        if (threadIdx.x < off)
-            sh[threadIdx.x] += sh[threadIdx.x + off];
-        __syncthreads();
-    }
-    const double r = sh[0];
-    __syncthreads();
-    return r;
-}
 
 struct PostArgs {
     DevCtl* ctl;
@@ -256,9 +239,11 @@ struct OpPost {
                 a.ctl->rebuild = 0;
             return;
         }
-        const double mv2 = block_fixed_sum(a.ke_partials, a.nb, 1);
+        double sum[1];
+        block_fixed_sums<1>(a.ke_partials, a.nb, 1, sum);
         if (threadIdx.x != 0)
             return;
+        const double mv2 = sum[0];
         DevCtl* c = a.ctl;
         const double ke = 0.5 * mass_v2_to_energy * mv2;
         double scale = 1.0;
@@ -307,8 +292,7 @@ struct OpKinStressSum {
     using Args = KinStressArgs;
     static __device__ void run(const KinStressArgs& a, int, int) {
         double v[6];
-        for (int c = 0; c < 6; ++c)
-            v[c] = block_fixed_sum(a.partials + 1 + c, a.nb, kPartialStride);
+        block_fixed_sums<6>(a.partials + 1, a.nb, kPartialStride, v);
         if (threadIdx.x == 0)
             for (int c = 0; c < 6; ++c)
                 a.ctl->stress_kin[c] = mass_v2_to_energy * v[c];
@@ -333,10 +317,8 @@ struct OpFinalize {
     using Args = FinalizeArgs;
     static __device__ void run(const FinalizeArgs& a, int, int) {
         double v[7], k[7];
-        for (int c = 0; c < 7; ++c)
-            v[c] = a.nb > 0 ? block_fixed_sum(a.partials + c, a.nb, kPartialStride) : 0.0;
-        for (int c = 0; c < 7; ++c)
-            k[c] = a.knb > 0 ? block_fixed_sum(a.kpartials + c, a.knb, kPartialStride) : 0.0;
+        block_fixed_sums<7>(a.partials, a.nb, kPartialStride, v);
+        block_fixed_sums<7>(a.kpartials, a.knb, kPartialStride, k);
         if (threadIdx.x == 0) {
             double pe = v[0];
             if (a.knb > 0) {
@@ -523,7 +505,8 @@ void md_enqueue_steps(atvh_system* s, int first, int nsteps, int precision, int 
             nl_enqueue_rebuild(s, &s->ctl->rebuild, false);
         }
         const bool ef = (step == nsteps - 1) || (energy_every > 0 && (step % energy_every) == 0);
-        pair_enqueue(s, precision, ef, ef);
+        // the virial is not recorded per step: only the last one can be read
+        pair_enqueue(s, precision, ef, step == nsteps - 1);
         if (ef)
             energy_enqueue_finalize(s, rec_pe, step);
         {

@@ -219,25 +219,16 @@ __global__ __launch_bounds__(kBlock) void k_npt_scale(NptArgs a) {
 
 // One block: column sums over the grid's partials, in block order, into
 // ctl->red; also clears the displacement flag ahead of the drift kernel.
-__global__ __launch_bounds__(kBlock) void k_npt_sum(const double* partials, int nb, int cols, DevCtl* ctl) {
-    __shared__ double sh[kBlock];
-    for (int c = 0; c < cols; ++c) {
-        double t = 0.0;
-        for (int b = threadIdx.x; b < nb; b += kBlock)
-            t += partials[(size_t)b * kPartialStride + c];
-        sh[threadIdx.x] = t;
-        __syncthreads();
-        for (int off = kBlock / 2; off > 0; off >>= 1) {
-            if (threadIdx.x < off)
-                sh[threadIdx.x] += sh[threadIdx.x + off];
-            __syncthreads();
-        }
-        if (threadIdx.x == 0)
-            ctl->red[c] = sh[0];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0)
+template <int kCols>
+__global__ __launch_bounds__(kBlock) void k_npt_sum(const double* partials, int nb, DevCtl* ctl) {
+    double v[kCols];
+    block_fixed_sums<kCols>(partials, nb, kPartialStride, v);
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int c = 0; c < kCols; ++c)
+            ctl->red[c] = v[c];
         ctl->disp_flag = 0;
+    }
 }
 
 int npt_grid(const atvh_system* s) { return std::min(grid_for(s->n), 1024); }
@@ -282,8 +273,9 @@ NptArgs npt_args(atvh_system* s) {
     return a;
 }
 
-void reduce(atvh_system* s, const NptArgs& a, int cols) {
-    k_npt_sum<<<1, kBlock, 0, s->ctx->stream>>>(a.partials, a.nb, cols, s->ctl);
+template <int kCols>
+void reduce(atvh_system* s, const NptArgs& a) {
+    k_npt_sum<kCols><<<1, kBlock, 0, s->ctx->stream>>>(a.partials, a.nb, s->ctl);
     ATVH_HIP(hipGetLastError());
 }
 
@@ -479,7 +471,7 @@ void npt_initial(atvh_system* s, NptState& q) {
         k_npt_chain_scale<<<a.nb, kBlock, 0, s->ctx->stream>>>(a);
         ATVH_HIP(hipGetLastError());
     }
-    reduce(s, a, 3);
+    reduce<3>(s, a);
     DevCtl h{};
     read_ctl(s, h);
     atoms_chain_forward(s, q, half_dt); // P2: forward sweep
@@ -538,7 +530,7 @@ double npt_final_end(atvh_system* s, NptState& q) {
         k_npt_kick_scale<<<a.nb, kBlock, 0, s->ctx->stream>>>(a);
         ATVH_HIP(hipGetLastError());
     }
-    reduce(s, a, 5);
+    reduce<5>(s, a);
     DevCtl h{};
     read_ctl(s, h);
     for (int d = 0; d < 3; ++d)

@@ -38,6 +38,41 @@ __device__ __forceinline__ void block_partials(double (&acc)[7], double* partial
     }
 }
 
+// Fixed-order sums of C columns over nb partial rows of `stride` doubles, by
+// one kBlock-thread block: thread t adds rows t, t + kBlock, ..., then the
+// threads are added in halves (t + 128, t + 64, ..., t + 1). Valid on thread
+// 0. One pass over the rows for all columns, the halves below a wavefront by
+// shuffles, one barrier (a pass and eight barriers per column before: energy
+// and virial of 2,048,000 atoms, 8,575 rows, 44 -> 11 us).
+template <int C>
+__device__ __forceinline__ void block_fixed_sums(const double* __restrict__ p, int nb, int stride, double (&out)[C]) {
+    __shared__ double sh[C][kBlock];
+    double t[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+        t[c] = 0.0;
+#pragma unroll 4
+    for (int b = threadIdx.x; b < nb; b += kBlock)
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+            t[c] += p[(int64_t)b * stride + c];
+    __syncthreads(); // sh may still be read by an earlier call
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+        sh[c][threadIdx.x] = t[c];
+    __syncthreads();
+    if (threadIdx.x >= 64)
+        return;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const double* s = sh[c] + threadIdx.x;
+        double v = (s[0] + s[128]) + (s[64] + s[192]);
+        for (int off = 32; off > 0; off >>= 1)
+            v += __shfl_down(v, off, 64);
+        out[c] = v;
+    }
+}
+
 // Image position of a halo row: the global slot's position plus the periodic
 // shift recorded at the build (positions are not re-wrapped between builds).
 __device__ __forceinline__ void row_image(const double* __restrict__ x, const double* __restrict__ y,

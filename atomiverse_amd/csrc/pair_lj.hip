@@ -642,7 +642,7 @@ void pair_enqueue(atvh_system* s, int precision, bool eflag, bool vflag) {
         lj_enqueue(s, precision, eflag, vflag); // times its own launch
     }
     if (s->pme)
-        pme_enqueue(s, precision, eflag || vflag);
+        pme_enqueue(s, precision, vflag ? 2 : (eflag ? 1 : 0));
 }
 
 static LJArgs lj_args(atvh_system* s) {
@@ -806,27 +806,25 @@ static void pair_batch_one(atvh_batch* b) {
                                                                          st.owner);
 }
 
-void pair_batch_launch(atvh_batch* b, int precision, bool ef) {
+template <template <bool, bool, bool> class OP>
+static void pair_batch_dispatch(atvh_batch* b, bool ef, bool vf) {
+    if (vf)
+        b->typed ? pair_batch_one<OP<true, true, true>>(b) : pair_batch_one<OP<true, true, false>>(b);
+    else if (ef)
+        b->typed ? pair_batch_one<OP<true, false, true>>(b) : pair_batch_one<OP<true, false, false>>(b);
+    else
+        b->typed ? pair_batch_one<OP<false, false, true>>(b) : pair_batch_one<OP<false, false, false>>(b);
+}
+
+void pair_batch_launch(atvh_batch* b, int precision, bool ef, bool vf) {
     for (atvh_system* s : b->solo)
-        pair_enqueue(s, precision, ef, ef);
+        pair_enqueue(s, precision, ef, vf);
     if (b->stages.find("pair") == b->stages.end())
         return;
-    const bool mixed = precision == ATVH_PREC_MIXED;
-    if (mixed) {
-        if (ef)
-            b->typed ? pair_batch_one<OpLjBrickMixed<true, true, true>>(b)
-                     : pair_batch_one<OpLjBrickMixed<true, true, false>>(b);
-        else
-            b->typed ? pair_batch_one<OpLjBrickMixed<false, false, true>>(b)
-                     : pair_batch_one<OpLjBrickMixed<false, false, false>>(b);
-    } else {
-        if (ef)
-            b->typed ? pair_batch_one<OpLjBrickFp64<true, true, true>>(b)
-                     : pair_batch_one<OpLjBrickFp64<true, true, false>>(b);
-        else
-            b->typed ? pair_batch_one<OpLjBrickFp64<false, false, true>>(b)
-                     : pair_batch_one<OpLjBrickFp64<false, false, false>>(b);
-    }
+    if (precision == ATVH_PREC_MIXED)
+        pair_batch_dispatch<OpLjBrickMixed>(b, ef, vf);
+    else
+        pair_batch_dispatch<OpLjBrickFp64>(b, ef, vf);
     ATVH_HIP(hipGetLastError());
 }
 

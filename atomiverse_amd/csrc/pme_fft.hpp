@@ -331,7 +331,8 @@ __global__ __launch_bounds__(kFftTileThreads) void k_fft_y(FftArgs a) {
 // inverse (decimation in time: bit-reversed in, natural out). Element e of a
 // tile is (j = e / kFftTile, column e % kFftTile) throughout; the next tile
 // and this tile's influence values are loaded while the current one works.
-template <class T, int LOG2N, bool EV>
+// EV: 0 none, 1 energy, 2 energy and virial.
+template <class T, int LOG2N, int EV>
 __global__ __launch_bounds__(kFftTileThreads) void k_fft_x_influence(FftArgs a) {
     using T2 = typename Cplx<T>::type;
     constexpr int N = 1 << LOG2N;
@@ -399,29 +400,30 @@ __global__ __launch_bounds__(kFftTileThreads) void k_fft_x_influence(FftArgs a) 
             const double h = hv[k];
             T2 v = buf[col][p];
             if (EV && h != 0.0) {
-                const int h0 = (m0 <= a.K0 / 2) ? m0 : m0 - a.K0;
-                const int h1 = (m1 <= a.K1 / 2) ? m1 : m1 - a.K1;
-                const int h2 = (m2 <= a.K2 / 2) ? m2 : m2 - a.K2;
-                const double mx = h0 * a.ic0, my = h1 * a.ic1, mz = h2 * a.ic2;
-                const double msq = mx * mx + my * my + mz * mz;
                 const double re = static_cast<double>(v.x), im = static_cast<double>(v.y);
-                const double q2 = re * re + im * im;
-                const double vt = -2.0 * (1.0 / msq + a.pi2_a2);
-                const double ug = h * q2;
+                const double ug = h * (re * re + im * im);
                 const bool pair = m2 != 0 && 2 * m2 != a.K2;
                 const double w = pair ? 2.0 : 1.0;
-                const double sx = (2 * m0 == a.K0) ? 1.0 : -1.0;
-                const double sy = (2 * m1 == a.K1) ? 1.0 : -1.0;
-                const double oxy = pair ? 1.0 + sx * sy : 1.0;
-                const double oxz = pair ? 1.0 - sx : 1.0;
-                const double oyz = pair ? 1.0 - sy : 1.0;
                 acc[0] += w * ug;
-                acc[1] += w * ug * (1.0 + vt * mx * mx);
-                acc[2] += w * ug * (1.0 + vt * my * my);
-                acc[3] += w * ug * (1.0 + vt * mz * mz);
-                acc[4] += oxy * ug * (vt * mx * my);
-                acc[5] += oxz * ug * (vt * mx * mz);
-                acc[6] += oyz * ug * (vt * my * mz);
+                if (EV == 2) {
+                    const int h0 = (m0 <= a.K0 / 2) ? m0 : m0 - a.K0;
+                    const int h1 = (m1 <= a.K1 / 2) ? m1 : m1 - a.K1;
+                    const int h2 = (m2 <= a.K2 / 2) ? m2 : m2 - a.K2;
+                    const double mx = h0 * a.ic0, my = h1 * a.ic1, mz = h2 * a.ic2;
+                    const double msq = mx * mx + my * my + mz * mz;
+                    const double vt = -2.0 * (1.0 / msq + a.pi2_a2);
+                    const double sx = (2 * m0 == a.K0) ? 1.0 : -1.0;
+                    const double sy = (2 * m1 == a.K1) ? 1.0 : -1.0;
+                    const double oxy = pair ? 1.0 + sx * sy : 1.0;
+                    const double oxz = pair ? 1.0 - sx : 1.0;
+                    const double oyz = pair ? 1.0 - sy : 1.0;
+                    acc[1] += w * ug * (1.0 + vt * mx * mx);
+                    acc[2] += w * ug * (1.0 + vt * my * my);
+                    acc[3] += w * ug * (1.0 + vt * mz * mz);
+                    acc[4] += oxy * ug * (vt * mx * my);
+                    acc[5] += oxz * ug * (vt * mx * mz);
+                    acc[6] += oyz * ug * (vt * my * mz);
+                }
             }
             v.x *= static_cast<T>(h);
             v.y *= static_cast<T>(h);
