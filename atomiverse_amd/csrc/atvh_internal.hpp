@@ -43,6 +43,7 @@ struct Error : std::runtime_error {
 // during a run; the host reads it at synchronisation points.
 struct DevCtl {
     double xi;        // Nose-Hoover thermostat variable
+    double xi_mid;    // xi between the two halves of a step (mid_enqueue_first_half)
     double nh_scale;  // NH velocity scale not yet applied to v (lazy)
     double pe;        // last potential energy
     double vir[6];    // last pair virial (Voigt xx yy zz xy xz yz)
@@ -342,6 +343,12 @@ void nl_check_ctl(const DevCtl& h);
 // rebuild counter keeps the rebuild the device already counted).
 void nl_build(atvh_system* s, bool keep_counts);
 
+// the list build of a rebuild whose sort and halo tables are done (brick layout)
+void nl_enqueue_pairs(atvh_system* s, const int* pred);
+// the permutation (from s->perm, keys in s->acell_of), halo tables and list
+// build after a sort that left the arrays in their old order
+void nl_enqueue_place(atvh_system* s);
+
 // pair_lj.hip
 int pair_grid(const atvh_system* s);
 void pair_enqueue(atvh_system* s, int precision, bool eflag, bool vflag);
@@ -400,6 +407,18 @@ struct ThermoRec {
 ThermoRec thermo_rec(atvh_system* s); // the system's own per-step record
 void md_enqueue_steps(atvh_system* s, int first, int nsteps, int precision, int energy_every, bool resume,
                       ThermoRec rec);
+// small_step.hip: whether one workgroup takes this system's integration and
+// sort, and that launch: the second half of step `final_step` (< 0: none; its
+// energy totals first when final_energy), then, when initial, the first half of
+// the next step up to a rebuild's halo tables.
+bool small_step_fits(const atvh_system* s);
+void small_enqueue_head(atvh_system* s, int final_step, bool final_energy, bool initial, ThermoRec rec);
+// small_step.hip: the same for systems of some tens of thousand atoms, the
+// atoms spread over blocks and the sort in one workgroup: the NH half of
+// `final_step` (whose kick is done), then the next step's first half and its
+// rebuild, list included.
+bool mid_step_fits(const atvh_system* s);
+void mid_enqueue_first_half(atvh_system* s, int final_step, bool final_energy, ThermoRec rec);
 // Regrow the list of a system halted by an overflow and finish its run alone
 // (bit-identical to the batched step); returns after the stream drains.
 void md_recover_and_finish(atvh_system* s, int nsteps, int precision, int energy_every);

@@ -57,6 +57,8 @@ struct BrickGeom {
     int max_atoms;              // home atoms the build takes per brick
 };
 
+BrickGeom brick_geom(const atvh_system* s); // neighbor.hip
+
 struct HaloTable {
     int dims[3];   // halo cells per axis
     int o[3];      // brick origin (cells)

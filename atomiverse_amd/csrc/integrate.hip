@@ -22,6 +22,7 @@
 
 #include "atvh_internal.hpp"
 #include "batch.hpp"
+#include "integrate.hpp"
 #include "pair_common.hpp"
 
 #include <algorithm>
@@ -35,86 +36,6 @@ using namespace atvh;
 namespace {
 
 constexpr int kIntGrid = 1024; // integrator grid cap: few kinetic partials to reduce
-
-struct IntArgs {
-    int64_t n;
-    double *x, *y, *z, *vx, *vy, *vz;
-    const double *fx, *fy, *fz;
-    const int* type;
-    const double *xs, *ys, *zs;
-    double dtfm[kMaxTypes];
-    double mass[kMaxTypes];
-    int ntypes;
-    double dt;
-    double lx, ly, lz;
-    double skin_sq;
-    int thermostat;
-    DevCtl* ctl;
-    double* ke_partials;
-};
-
-__device__ __forceinline__ double wave_sum_d(double v) {
-    for (int off = 32; off > 0; off >>= 1)
-        v += __shfl_down(v, off, 64);
-    return v;
-}
-
-__device__ __forceinline__ void block_sum_to(double v, double* out) {
-    __shared__ double sh[kBlock / 64];
-    v = wave_sum_d(v);
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    if (lane == 0)
-        sh[wid] = v;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double t = 0.0;
-        for (int w = 0; w < kBlock / 64; ++w)
-            t += sh[w];
-        *out = t;
-    }
-}
-
-// The kicks: one atom per grid-stride step, its loads issued before its
-// stores. A one-type frame takes dtfm and mass from scalars (no dependent
-// per-atom table loads). (Two atoms per step, both loaded before either is
-// stored, needed 142 registers for the initial kick and lost on the batched
-// ladder what it gained on the 2.048M-atom fluid.)
-struct KickAtom {
-    double vx, vy, vz, fx, fy, fz;
-    int t;
-};
-
-__device__ __forceinline__ KickAtom kick_load(const IntArgs& a, int64_t i, bool typed) {
-    KickAtom k;
-    k.t = typed ? a.type[i] : 0;
-    k.vx = a.vx[i];
-    k.vy = a.vy[i];
-    k.vz = a.vz[i];
-    k.fx = a.fx[i];
-    k.fy = a.fy[i];
-    k.fz = a.fz[i];
-    return k;
-}
-
-// v <- (v s) + dtfm f (the reference's order: the pending NH scale, then the
-// kick); returns m v^2 of the new velocity
-__device__ __forceinline__ double kick_apply(const IntArgs& a, KickAtom& k, double s, bool typed, double dtfm0,
-                                             double m0) {
-    double dtfm = dtfm0, m = m0;
-    if (typed) {
-        dtfm = a.dtfm[k.t];
-        m = a.mass[k.t];
-    }
-    if (a.thermostat) {
-        k.vx *= s;
-        k.vy *= s;
-        k.vz *= s;
-    }
-    k.vx += dtfm * k.fx;
-    k.vy += dtfm * k.fy;
-    k.vz += dtfm * k.fz;
-    return m * (k.vx * k.vx + k.vy * k.vy + k.vz * k.vz);
-}
 
 struct OpInitial {
     using Args = IntArgs;
@@ -140,12 +61,7 @@ struct OpInitial {
         a.vx[i] = k.vx;
         a.vy[i] = k.vy;
         a.vz[i] = k.vz;
-        double dx = x - p.xs, dy = y - p.ys, dz = z - p.zs;
-        dx -= a.lx * nearbyint(dx / a.lx);
-        dy -= a.ly * nearbyint(dy / a.ly);
-        dz -= a.lz * nearbyint(dz / a.lz);
-        const double dsq = dx * dx + dy * dy + dz * dz;
-        if (dsq * 4.0 > a.skin_sq)
+        if (moved_past_skin(a, x - p.xs, y - p.ys, z - p.zs))
             moved = 1;
     }
     static __device__ void run(const IntArgs& a, int bid, int nbk) {
@@ -249,8 +165,9 @@ struct OpPost {
         double scale = 1.0;
         if (a.thermostat) {
             // Q and Ndof kB T live in the control block (a replica exchange moves them)
-            c->xi += (a.dt * 0.5) * (2.0 * ke - c->nh_ndof_kT) / c->nh_Q;
-            scale = exp(-a.dt * 0.5 * c->xi);
+            double xi = c->xi;
+            scale = nh_update(ke, a.dt, c->nh_ndof_kT, c->nh_Q, xi);
+            c->xi = xi;
             c->nh_scale = scale;
         }
         if (a.final_phase) {
@@ -264,20 +181,8 @@ struct OpPost {
         } else {
             c->ke_half = ke;
         }
-        if (a.decide) {
-            c->ago += 1;
-            const bool delay_ok = c->ago >= a.delay;
-            const bool every_ok = (c->ago % a.every) == 0;
-            const bool rb = delay_ok && every_ok && (!a.check || c->disp_flag != 0);
-            c->disp_flag = 0;
-            c->rebuild = rb ? 1 : 0;
-            if (rb) {
-                c->ago = 0;
-                c->nrebuilds += 1;
-                c->nbr_total = 0;
-                c->max_nbr = 0;
-            }
-        }
+        if (a.decide)
+            decide_reneighbor(c, a.every, a.delay, a.check, c->disp_flag != 0);
     }
 };
 
@@ -299,45 +204,9 @@ struct OpKinStressSum {
     }
 };
 
-struct FinalizeArgs {
-    DevCtl* ctl;
-    const double* partials; // pair style, per workgroup
-    int nb;
-    const double* kpartials; // k-space influence, per workgroup (kspace only)
-    int knb;
-    double escale, e_self, e_net;
-    double* record_pe;
-    int step; // record index; < 0: the device counter ctl->rec_step
-};
-
-// Fixed-order totals of the force phase: pair energy and virial, then the
-// k-space terms in the reference's order (self first, then reciprocal + net
-// charge; pme.cpp:222-246).
 struct OpFinalize {
     using Args = FinalizeArgs;
-    static __device__ void run(const FinalizeArgs& a, int, int) {
-        double v[7], k[7];
-        block_fixed_sums<7>(a.partials, a.nb, kPartialStride, v);
-        block_fixed_sums<7>(a.kpartials, a.knb, kPartialStride, k);
-        if (threadIdx.x == 0) {
-            double pe = v[0];
-            if (a.knb > 0) {
-                const double e_recip = k[0] * a.escale;
-                pe += a.e_self;
-                pe += e_recip + a.e_net;
-                for (int c = 0; c < 6; ++c)
-                    v[c + 1] += k[c + 1] * a.escale;
-                a.ctl->e_kspace[0] = e_recip;
-                a.ctl->e_kspace[1] = a.e_self;
-                a.ctl->e_kspace[2] = a.e_net;
-            }
-            a.ctl->pe = pe;
-            for (int c = 0; c < 6; ++c)
-                a.ctl->vir[c] = v[c + 1];
-            if (a.record_pe)
-                a.record_pe[a.step >= 0 ? a.step : a.ctl->rec_step] = pe;
-        }
-    }
+    static __device__ void run(const FinalizeArgs& a, int, int) { finalize_totals(a); }
 };
 
 // Start of a fused run: no step of it completed yet.
@@ -345,6 +214,32 @@ __global__ void k_run_reset(DevCtl* ctl) {
     if (threadIdx.x == 0 && blockIdx.x == 0)
         ctl->steps_done = 0;
 }
+
+PostArgs make_post_args(atvh_system* s, bool final_phase, bool decide) {
+    PostArgs p{};
+    p.ctl = s->ctl;
+    p.ke_partials = ke_partials_of(s, 0);
+    p.nb = std::min(grid_for(s->n), kIntGrid);
+    p.thermostat = s->thermostat;
+    p.dt = s->dt;
+    p.decide = decide ? 1 : 0;
+    p.every = s->every;
+    p.delay = s->delay;
+    p.check = s->check;
+    p.record_ke = nullptr;
+    p.step = 0;
+    p.final_phase = final_phase ? 1 : 0;
+    return p;
+}
+
+void check_integ(atvh_system* s) {
+    if (!s->integ_configured)
+        throw Error(ATVH_E_STATE, "integrator not configured");
+}
+
+} // namespace
+
+namespace atvh {
 
 IntArgs make_int_args(atvh_system* s) {
     IntArgs a{};
@@ -376,35 +271,9 @@ IntArgs make_int_args(atvh_system* s) {
     a.skin_sq = s->skin * s->skin;
     a.thermostat = s->thermostat;
     a.ctl = s->ctl;
-    a.ke_partials = s->partials + size_t(s->npartials) * kPartialStride;
+    a.ke_partials = ke_partials_of(s, 0);
     return a;
 }
-
-PostArgs make_post_args(atvh_system* s, bool final_phase, bool decide) {
-    PostArgs p{};
-    p.ctl = s->ctl;
-    p.ke_partials = s->partials + size_t(s->npartials) * kPartialStride;
-    p.nb = std::min(grid_for(s->n), kIntGrid);
-    p.thermostat = s->thermostat;
-    p.dt = s->dt;
-    p.decide = decide ? 1 : 0;
-    p.every = s->every;
-    p.delay = s->delay;
-    p.check = s->check;
-    p.record_ke = nullptr;
-    p.step = 0;
-    p.final_phase = final_phase ? 1 : 0;
-    return p;
-}
-
-void check_integ(atvh_system* s) {
-    if (!s->integ_configured)
-        throw Error(ATVH_E_STATE, "integrator not configured");
-}
-
-} // namespace
-
-namespace atvh {
 
 int integ_grid(const atvh_system* s) { return std::min(grid_for(s->n), kIntGrid); }
 
@@ -490,7 +359,37 @@ void md_enqueue_steps(atvh_system* s, int first, int nsteps, int precision, int 
     hipStream_t st = c->stream;
     double* rec_pe = rec.pe;
     double* rec_ke = rec.ke;
+    const auto energy_step = [&](int step) {
+        return step == nsteps - 1 || (energy_every > 0 && step % energy_every == 0);
+    };
     const IntArgs ia = make_int_args(s);
+    if (small_step_fits(s)) {
+        // one workgroup holds the whole integration, decision and sort: step
+        // k's second half and step k + 1's first half share a launch
+        for (int step = first; step < nsteps; ++step) {
+            if (!(resume && step == first)) {
+                small_enqueue_head(s, step > first ? step - 1 : -1, energy_step(step - 1), true, rec);
+                nl_enqueue_pairs(s, &s->ctl->rebuild);
+            }
+            pair_enqueue(s, precision, energy_step(step), step == nsteps - 1);
+        }
+        if (nsteps > first)
+            small_enqueue_head(s, nsteps - 1, true, false, rec);
+        return;
+    }
+    if (mid_step_fits(s)) {
+        for (int step = first; step < nsteps; ++step) {
+            if (!(resume && step == first))
+                mid_enqueue_first_half(s, step > first ? step - 1 : -1, energy_step(step - 1), rec);
+            pair_enqueue(s, precision, energy_step(step), step == nsteps - 1);
+            enqueue_final_kick(s, ia);
+        }
+        if (nsteps > first) {
+            energy_enqueue_finalize(s, rec_pe, nsteps - 1);
+            enqueue_final_post(s, nsteps - 1, rec);
+        }
+        return;
+    }
     PostArgs p_init = make_post_args(s, false, true);
     PostArgs p_fin = make_post_args(s, true, false);
     p_fin.record_ke = rec_ke;
@@ -504,7 +403,7 @@ void md_enqueue_steps(atvh_system* s, int first, int nsteps, int precision, int 
             k_single<OpPost><<<1, kBlock, 0, st>>>(p_init);
             nl_enqueue_rebuild(s, &s->ctl->rebuild, false);
         }
-        const bool ef = (step == nsteps - 1) || (energy_every > 0 && (step % energy_every) == 0);
+        const bool ef = energy_step(step);
         // the virial is not recorded per step: only the last one can be read
         pair_enqueue(s, precision, ef, step == nsteps - 1);
         if (ef)
@@ -540,7 +439,25 @@ void md_recover_and_finish(atvh_system* s, int nsteps, int precision, int energy
     }
 }
 
-void energy_enqueue_finalize(atvh_system* s, double* record_pe, int step, bool with_pair) {
+void enqueue_final_kick(atvh_system* s, const IntArgs& a) {
+    ScopedTimer tm(s->ctx, "integrate");
+    k_single<OpFinal><<<integ_grid(s), kBlock, 0, s->ctx->stream>>>(a);
+    ATVH_HIP(hipGetLastError());
+}
+
+void enqueue_final_post(atvh_system* s, int step, ThermoRec rec) {
+    PostArgs p = make_post_args(s, true, false);
+    p.record_ke = rec.ke;
+    p.step = step;
+    k_single<OpPost><<<1, kBlock, 0, s->ctx->stream>>>(p);
+    ATVH_HIP(hipGetLastError());
+}
+
+double* ke_partials_of(const atvh_system* s, int which) {
+    return s->partials + size_t(s->npartials) * kPartialStride + size_t(which) * kIntGrid;
+}
+
+FinalizeArgs make_finalize_args(atvh_system* s, double* record_pe, int step, bool with_pair) {
     FinalizeArgs a{};
     a.ctl = s->ctl;
     a.partials = s->partials;
@@ -552,6 +469,11 @@ void energy_enqueue_finalize(atvh_system* s, double* record_pe, int step, bool w
         pme_energy_consts(s, a.escale, a.e_self, a.e_net);
     a.record_pe = record_pe;
     a.step = step;
+    return a;
+}
+
+void energy_enqueue_finalize(atvh_system* s, double* record_pe, int step, bool with_pair) {
+    const FinalizeArgs a = make_finalize_args(s, record_pe, step, with_pair);
     k_single<OpFinalize><<<1, kBlock, 0, s->ctx->stream>>>(a);
     ATVH_HIP(hipGetLastError());
 }

@@ -28,6 +28,7 @@
 #include "atvh_internal.hpp"
 #include "batch.hpp"
 #include "brick.hpp"
+#include "pair_common.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -680,18 +681,6 @@ __device__ __forceinline__ bool band_pair_args(const BrickBuildArgs& ab, const i
     return band_pair(ab.x, ab.y, ab.z, ab.rc_sq, g.L[0], g.L[1], g.L[2], g.nc[0], g.nc[1], g.nc[2], h_off, ncell, HY,
                      HZ, q, lx + g.R[0], ly + g.R[1], lz + g.R[2], o0 + lx, o1 + ly, o2 + lz, gi,
                      rows[q] & kRowSlotMask);
-}
-
-// Inclusive prefix sum over the 64 lanes (DPP row shifts, then the row
-// broadcasts of lanes 15 and 31).
-__device__ __forceinline__ int wave_inclusive_sum(int x) {
-    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true); // row_shr:1
-    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true); // row_shr:2
-    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true); // row_shr:4
-    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true); // row_shr:8
-    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false); // row_bcast:15 -> rows 1, 3
-    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false); // row_bcast:31 -> rows 2, 3
-    return x;
 }
 
 struct OpPairs {
@@ -1700,6 +1689,141 @@ void nl_enqueue_rebuild(atvh_system* s, const int* pred, bool permute_forces) {
                      s->nbr, s->numneigh, s->cap, s->npad, s->ctl};
         k_nl_build_small<<<grid_capped(s->n, kBlock / 64), kBlock, 0, st>>>(pred, s->n, ba);
     }
+    ATVH_HIP(hipGetLastError());
+}
+
+void nl_enqueue_pairs(atvh_system* s, const int* pred) {
+    ScopedTimer tm(s->ctx, "nlist");
+    k_single<OpPairs><<<s->nbricks, OpPairs::kThreads, 0, s->ctx->stream>>>(nl_brick_args(s, pred));
+    ATVH_HIP(hipGetLastError());
+}
+
+// After mid_enqueue_first_half's sort (small_step.hip): perm lists the atoms
+// cell by cell in no order within a cell, the cell starts are final, the keys
+// (cell ranks) and every array are still in the old slot order. Blocks [0, gp)
+// gather each atom into the permutation scratch at its final place (the count
+// of smaller tags in its cell), the rest make the halo tables; the list build
+// then reads the scratch, and each of its workgroups first copies its brick's
+// own slots back to the system's arrays (a brick owns a slot range, and nobody
+// reads another brick's slots there in that launch), so no snapshot stage and
+// no separate copy back are launched.
+struct PlaceArgs {
+    BrickBuildArgs h;
+    int gp;
+    int64_t n;
+    const int *perm, *key, *start;
+    double lx, ly, lz;
+    const double *x, *y, *z, *vx, *vy, *vz, *q;
+    const int *tag, *type;
+    double *ox, *oy, *oz, *ovx, *ovy, *ovz, *oq, *xs, *ys, *zs;
+    int *otag, *otype;
+    int with_q, with_type;
+};
+
+struct OpPlaceHalo {
+    using Args = PlaceArgs;
+    static __device__ void run(const PlaceArgs& a, int bid, int nbk) {
+        if (!*a.h.pred)
+            return;
+        if (bid >= a.gp) {
+            OpHalo::run(a.h, bid - a.gp, nbk - a.gp);
+            return;
+        }
+        for (int64_t s = bid * (int64_t)blockDim.x + threadIdx.x; s < a.n; s += (int64_t)a.gp * blockDim.x) {
+            const int p = a.perm[s];
+            const int c = a.key[p], t = a.tag[p];
+            const int b = a.start[c], e = a.start[c + 1];
+            int d = b;
+            for (int k = b; k < e; ++k)
+                d += a.tag[a.perm[k]] < t ? 1 : 0;
+            double xi = a.x[p], yi = a.y[p], zi = a.z[p];
+            xi -= a.lx * floor(xi / a.lx); // wrap_orthorhombic at the rebuild (OpBin)
+            yi -= a.ly * floor(yi / a.ly);
+            zi -= a.lz * floor(zi / a.lz);
+            a.ox[d] = xi;
+            a.oy[d] = yi;
+            a.oz[d] = zi;
+            a.xs[d] = xi;
+            a.ys[d] = yi;
+            a.zs[d] = zi;
+            a.ovx[d] = a.vx[p];
+            a.ovy[d] = a.vy[p];
+            a.ovz[d] = a.vz[p];
+            a.otag[d] = t;
+            if (a.with_q)
+                a.oq[d] = a.q[p];
+            if (a.with_type)
+                a.otype[d] = a.type[p];
+        }
+    }
+};
+
+struct PairsCopyArgs {
+    BrickBuildArgs b; // first: the band test reads it at the start of the kernel-argument segment
+    const double *ox, *oy, *oz, *ovx, *ovy, *ovz, *oq;
+    const int *otag, *otype;
+    double *x, *y, *z, *vx, *vy, *vz, *q;
+    int *tag, *type;
+    int with_q, with_type;
+};
+
+struct OpPairsCopy {
+    using Args = PairsCopyArgs;
+    static constexpr int kThreads = OpPairs::kThreads;
+    static constexpr int kMinWaves = OpPairs::kMinWaves;
+    static __device__ void run(const PairsCopyArgs& a, int bid, int nbk) {
+        if (!*a.b.pred)
+            return;
+        const int2 br = a.b.brick_range[xcd_brick(bid, a.b.nbricks)];
+        for (int s = br.x + threadIdx.x; s < br.x + br.y; s += kThreads) {
+            a.x[s] = a.ox[s];
+            a.y[s] = a.oy[s];
+            a.z[s] = a.oz[s];
+            a.vx[s] = a.ovx[s];
+            a.vy[s] = a.ovy[s];
+            a.vz[s] = a.ovz[s];
+            a.tag[s] = a.otag[s];
+            if (a.with_q)
+                a.q[s] = a.oq[s];
+            if (a.with_type)
+                a.type[s] = a.otype[s];
+        }
+        OpPairs::run(a.b, bid, nbk);
+    }
+};
+
+void nl_enqueue_place(atvh_system* s) {
+    ScopedTimer tm(s->ctx, "nlist");
+    hipStream_t st = s->ctx->stream;
+    PairsCopyArgs c{};
+    c.b = nl_brick_args(s, &s->ctl->rebuild);
+    c.b.x = s->ax;
+    c.b.y = s->ay;
+    c.b.z = s->az;
+    PlaceArgs p{};
+    p.h = c.b;
+    p.n = s->n;
+    p.perm = s->perm;
+    p.key = s->acell_of;
+    p.start = s->cell_start;
+    p.lx = s->box[0];
+    p.ly = s->box[1];
+    p.lz = s->box[2];
+    c.x = s->x, c.y = s->y, c.z = s->z, c.vx = s->vx, c.vy = s->vy, c.vz = s->vz, c.q = s->q;
+    p.x = s->x, p.y = s->y, p.z = s->z, p.vx = s->vx, p.vy = s->vy, p.vz = s->vz, p.q = s->q;
+    c.ox = p.ox = s->ax, c.oy = p.oy = s->ay, c.oz = p.oz = s->az;
+    c.ovx = p.ovx = s->avx, c.ovy = p.ovy = s->avy, c.ovz = p.ovz = s->avz;
+    c.oq = p.oq = s->aq;
+    p.xs = s->xs, p.ys = s->ys, p.zs = s->zs;
+    c.tag = s->tag, c.type = s->type;
+    p.tag = s->tag, p.type = s->type;
+    c.otag = p.otag = s->atag;
+    c.otype = p.otype = s->atype;
+    c.with_q = p.with_q = s->has_charge ? 1 : 0;
+    c.with_type = p.with_type = s->ntypes > 1 ? 1 : 0;
+    p.gp = grid_for(s->n);
+    k_single<OpPlaceHalo><<<p.gp + s->nbricks, kBlock, 0, st>>>(p);
+    k_single<OpPairsCopy><<<s->nbricks, OpPairsCopy::kThreads, 0, st>>>(c);
     ATVH_HIP(hipGetLastError());
 }
 

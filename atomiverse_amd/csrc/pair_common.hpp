@@ -40,8 +40,8 @@ __device__ __forceinline__ void block_partials(double (&acc)[7], double* partial
 
 // Fixed-order sums of C columns over nb partial rows of `stride` doubles, by
 // one kBlock-thread block: thread t adds rows t, t + kBlock, ..., then the
-// threads are added in halves (t + 128, t + 64, ..., t + 1). Valid on thread
-// 0. One pass over the rows for all columns, the halves below a wavefront by
+// threads are added in halves (t + 128, t + 64, ..., t + 1); threads past
+// kBlock of a larger block only meet the barriers. Valid on thread 0. One pass over the rows for all columns, the halves below a wavefront by
 // shuffles, one barrier (a pass and eight barriers per column before: energy
 // and virial of 2,048,000 atoms, 8,575 rows, 44 -> 11 us).
 template <int C>
@@ -51,15 +51,17 @@ __device__ __forceinline__ void block_fixed_sums(const double* __restrict__ p, i
 #pragma unroll
     for (int c = 0; c < C; ++c)
         t[c] = 0.0;
+    if (threadIdx.x < kBlock)
 #pragma unroll 4
-    for (int b = threadIdx.x; b < nb; b += kBlock)
+        for (int b = threadIdx.x; b < nb; b += kBlock)
+#pragma unroll
+            for (int c = 0; c < C; ++c)
+                t[c] += p[(int64_t)b * stride + c];
+    __syncthreads(); // sh may still be read by an earlier call
+    if (threadIdx.x < kBlock)
 #pragma unroll
         for (int c = 0; c < C; ++c)
-            t[c] += p[(int64_t)b * stride + c];
-    __syncthreads(); // sh may still be read by an earlier call
-#pragma unroll
-    for (int c = 0; c < C; ++c)
-        sh[c][threadIdx.x] = t[c];
+            sh[c][threadIdx.x] = t[c];
     __syncthreads();
     if (threadIdx.x >= 64)
         return;
@@ -109,6 +111,18 @@ __device__ __forceinline__ void small_lane_sum(T& v) {
 #pragma unroll
     for (int off = kSmallLanes / 2; off > 0; off >>= 1)
         v += __shfl_xor(v, off, 64);
+}
+
+// Inclusive prefix sum over the 64 lanes (DPP row shifts, then the row
+// broadcasts of lanes 15 and 31).
+__device__ __forceinline__ int wave_inclusive_sum(int x) {
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true); // row_shr:1
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true); // row_shr:2
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true); // row_shr:4
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true); // row_shr:8
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false); // row_bcast:15 -> rows 1, 3
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false); // row_bcast:31 -> rows 2, 3
+    return x;
 }
 
 // Unpack entry u (0..7) of an 8-wide group of 16-bit halo rows.
