@@ -96,8 +96,16 @@ void fetch_pieces(atvh_ctx* c, const std::vector<HostPiece>& pieces) {
         total = runs.back().at + up(runs.back().bytes);
     }
     if (total > kStageMax) {
-        for (const HostPiece& q : pieces)
+        // three pageable copies in flight at most, none queued behind kernels:
+        // nine queued at once left the caller's next host threads stalled for
+        // 10-40 ms now and then (a 512,000-ion run's snapshots)
+        ATVH_HIP(hipStreamSynchronize(c->stream));
+        int queued = 0;
+        for (const HostPiece& q : pieces) {
             ATVH_HIP(hipMemcpyAsync(q.dst, q.src, q.bytes, hipMemcpyDeviceToHost, c->stream));
+            if (++queued % 3 == 0)
+                ATVH_HIP(hipStreamSynchronize(c->stream));
+        }
         ATVH_HIP(hipStreamSynchronize(c->stream));
         return;
     }
