@@ -313,6 +313,11 @@ void k_ljc_brick_mixed(LjcArgs a) {
     const int b = xcd_brick(blockIdx.x, gridDim.x); // one launch block per brick
     const int nh = a.halo_n[b];
     const int2 br = a.brick_range[b];
+    const int* __restrict__ rows = a.halo_rows + (int64_t)b * kHaloCap;
+    int row[kHaloCap / kLjcMixedThreads]; // this thread's halo rows (see AtomRow)
+#pragma unroll
+    for (int k = 0; k < kHaloCap / kLjcMixedThreads; ++k)
+        row[k] = rows[threadIdx.x + k * kLjcMixedThreads];
     const int a0 = br.x, nat = br.y;
     double acc[7] = {0, 0, 0, 0, 0, 0, 0};
     if (brick_skipped(nh, nat, a.max_atoms)) { // reported by the build; nothing valid to compute
@@ -320,20 +325,29 @@ void k_ljc_brick_mixed(LjcArgs a) {
             block_partials<kLjcMixedThreads>(acc, a.partials, blockIdx.x);
         return;
     }
-    const int* __restrict__ rows = a.halo_rows + (int64_t)b * kHaloCap;
     double r0x, r0y, r0z;
     brick_centre(b, a.nb, a.bdim, a.nc, a.cs, r0x, r0y, r0z);
-    for (int r = threadIdx.x; r < nh; r += blockDim.x) {
-        int gs;
-        double xx, yy, zz;
-        row_image(a.x, a.y, a.z, a.L[0], a.L[1], a.L[2], rows[r], gs, xx, yy, zz);
-        float4 v;
-        v.x = static_cast<float>(xx - r0x);
-        v.y = static_cast<float>(yy - r0y);
-        v.z = static_cast<float>(zz - r0z);
-        v.w = static_cast<float>(a.q[gs]);
-        sp[r] = v;
-        stype[r] = static_cast<unsigned char>(a.type[gs]);
+    // two threads per atom when the brick has at most half a block of atoms
+    const int tpa = (2 * nat <= kLjcMixedThreads) ? 2 : 1;
+    // (an empty brick may start past the last slot: its group loads read slot 0's)
+    const uint4* __restrict__ base = reinterpret_cast<const uint4*>(a.nbr16 + (int64_t)(nat > 0 ? a0 : 0) * a.cap);
+    int t = threadIdx.x;
+    AtomRow ar = atom_row(a.self16, a.numneigh, a0, nat, tpa, t);
+#pragma unroll
+    for (int k = 0; k < kHaloCap / kLjcMixedThreads; ++k) {
+        const int r = threadIdx.x + k * kLjcMixedThreads;
+        if (r < nh) {
+            int gs;
+            double xx, yy, zz;
+            row_image(a.x, a.y, a.z, a.L[0], a.L[1], a.L[2], row[k], gs, xx, yy, zz);
+            float4 v;
+            v.x = static_cast<float>(xx - r0x);
+            v.y = static_cast<float>(yy - r0y);
+            v.z = static_cast<float>(zz - r0z);
+            v.w = static_cast<float>(a.q[gs]);
+            sp[r] = v;
+            stype[r] = static_cast<unsigned char>(a.type[gs]);
+        }
     }
     if (threadIdx.x == 0) { // the list's padding row: out of every cutoff
         sp[kSentinelRow] = make_float4(kSentinelFarF, kSentinelFarF, kSentinelFarF, 0.0f);
@@ -342,30 +356,24 @@ void k_ljc_brick_mixed(LjcArgs a) {
     if (SMALLTAB)
         for (int k = threadIdx.x; k < a.ntypes * a.ntypes * 8; k += blockDim.x)
             ljt[(k / (a.ntypes * 8)) * kLjcLdsTypes * 8 + k % (a.ntypes * 8)] = a.tab32[k];
+    uint4 cur = base[group_at(ar, nat, 0, tpa)], nx1 = base[group_at(ar, nat, 1, tpa)];
     __syncthreads();
     const float rc_sq = static_cast<float>(a.rc_sq);
     const float alpha = static_cast<float>(a.alpha);
     const float two_a_rtpi = static_cast<float>(kEwaldF * a.alpha);
     const int ntypes = a.ntypes;
     const float* __restrict__ tab = a.tab32;
-    const uint4* __restrict__ base = reinterpret_cast<const uint4*>(a.nbr16 + (int64_t)a0 * a.cap);
-    // two threads per atom when the brick has at most half a block of atoms
-    const int tpa = (2 * nat <= static_cast<int>(blockDim.x)) ? 2 : 1;
-    for (int t = threadIdx.x; t < nat * tpa; t += blockDim.x) {
-        const int li = tpa == 2 ? (t >> 1) : t;
-        const int h = tpa == 2 ? (t & 1) : 0;
+    while (t < nat * tpa) {
+        const int li = ar.li, h = ar.h;
         const int i = a0 + li;
-        const int qs = a.self16[i];
+        const int qs = ar.qs;
         const float4 pi = sp[qs];
         const float qi_scale = static_cast<float>(coulomb) * pi.w;
         const float* __restrict__ trow = SMALLTAB ? ljt + stype[qs] * kLjcLdsTypes * 8 : tab + stype[qs] * ntypes * 8;
-        const int nn = a.numneigh[i];
         const uint4* __restrict__ grp = base + li;
-        const int ng = (nn + kGroup - 1) / kGroup;
+        const int ng = ar.ng;
         float fxi = 0.f, fyi = 0.f, fzi = 0.f;
-        const int gl = max(ng - 1, 0); // group 0 exists even when nn == 0
-        uint4 cur = grp[__umul24(min(h, gl), nat)];
-        uint4 nx1 = grp[__umul24(min(h + tpa, gl), nat)];
+        const int gl = max(ng - 1, 0); // group 0 exists even in an empty row
         for (int g = h; g < ng; g += tpa) {
             const uint4 nx2 = grp[__umul24(min(g + 2 * tpa, gl), nat)];
             // each half group's LDS reads issue before its arithmetic (half
@@ -428,11 +436,17 @@ void k_ljc_brick_mixed(LjcArgs a) {
             fyi += __shfl_xor(fyi, 1, 64);
             fzi += __shfl_xor(fzi, 1, 64);
         }
-        if (h != 0)
-            continue;
-        a.fx[i] = static_cast<double>(fxi);
-        a.fy[i] = static_cast<double>(fyi);
-        a.fz[i] = static_cast<double>(fzi);
+        if (h == 0) {
+            a.fx[i] = static_cast<double>(fxi);
+            a.fy[i] = static_cast<double>(fyi);
+            a.fz[i] = static_cast<double>(fzi);
+        }
+        t += kLjcMixedThreads;
+        if (t < nat * tpa) {
+            ar = atom_row(a.self16, a.numneigh, a0, nat, tpa, t);
+            cur = base[group_at(ar, nat, 0, tpa)];
+            nx1 = base[group_at(ar, nat, 1, tpa)];
+        }
     }
     if (EF || VF) {
 #pragma unroll

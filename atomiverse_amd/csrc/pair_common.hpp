@@ -98,6 +98,46 @@ __device__ __forceinline__ void brick_centre(int b, const int nb[3], const int b
     cz = (oz + 0.5 * min(bdim[2], nc[2] - oz)) * cs[2];
 }
 
+// What a thread of a brick pair kernel loads ahead of the halo barrier. The
+// kernels used to find the halo size, then the rows, then the positions, and
+// after the barrier the atom's row header, then its list: five dependent trips
+// to memory of ~1 us each before the first pair, most of a small system's
+// force call. The rows are read without waiting for the halo's size (the table
+// always holds kHaloCap entries; those past the halo are not used), and the
+// row header and first two list groups while the positions are on their way.
+struct AtomRow {
+    int li; // the atom, brick-local
+    int h;  // which of its threads this is
+    int qs; // its own halo row
+    int ng; // list groups
+};
+
+// Thread t's atom with tpa threads per atom (lanes 2l, 2l + 1 for tpa 2); a
+// thread past the brick's atoms takes the last one's row header and uses none
+// of it.
+__device__ __forceinline__ AtomRow atom_row(const uint16_t* __restrict__ self16, const int* __restrict__ numneigh,
+                                            int a0, int nat, int tpa, int t) {
+    AtomRow r;
+    r.li = tpa == 2 ? (t >> 1) : t;
+    r.h = tpa == 2 ? (t & 1) : 0;
+    r.qs = 0;
+    r.ng = 0;
+    if (r.li < nat) {
+        r.qs = self16[a0 + r.li];
+        r.ng = (numneigh[a0 + r.li] + kGroup - 1) / kGroup;
+    } else {
+        r.li = 0;
+    }
+    return r;
+}
+
+// Index (16-byte groups from the brick's list) of the k-th group of this
+// thread, clamped to the atom's last one (to group 0 of an empty row: the
+// brick's rows always exist while it has atoms).
+__device__ __forceinline__ int group_at(const AtomRow& r, int nat, int k, int tpa) {
+    return __umul24(min(r.h + k * tpa, max(r.ng - 1, 0)), nat) + r.li;
+}
+
 // Small-grid pair kernels: kSmallLanes consecutive lanes share an atom, lane k
 // taking entries k, k + kSmallLanes, ... of its row. Those systems are a few
 // hundred atoms (or a thin box), where one thread per atom is a serial chain

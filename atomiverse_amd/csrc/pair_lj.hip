@@ -358,6 +358,11 @@ __device__ void OpLjBrickMixed<EF, VF, TYPED>::run(const BrickLJArgs& a, int bid
     const int b = xcd_brick(bid, nbk); // one launch block per brick
     const int nh = a.halo_n[b];
     const int2 br = a.brick_range[b];
+    const int* __restrict__ rows = a.halo_rows + (int64_t)b * kHaloCap;
+    int row[kHaloCap / kThreads]; // this thread's halo rows (see AtomRow)
+#pragma unroll
+    for (int k = 0; k < kHaloCap / kThreads; ++k)
+        row[k] = rows[threadIdx.x + k * kThreads];
     const int a0 = br.x, nat = br.y;
     double acc[7] = {0, 0, 0, 0, 0, 0, 0};
     if (brick_skipped(nh, nat, a.max_atoms)) { // reported by the build; nothing valid to compute
@@ -365,7 +370,6 @@ __device__ void OpLjBrickMixed<EF, VF, TYPED>::run(const BrickLJArgs& a, int bid
             block_partials<kThreads>(acc, a.partials, bid);
         return;
     }
-    const int* __restrict__ rows = a.halo_rows + (int64_t)b * kHaloCap;
     // reference point: the brick centre (every halo row lies within the brick
     // widened by the stencil reach, so |x - centre| < ~7 Å and the FP32
     // rounding of the relative coordinate is <= 2.4e-7 Å)
@@ -376,26 +380,37 @@ __device__ void OpLjBrickMixed<EF, VF, TYPED>::run(const BrickLJArgs& a, int bid
     double r0x, r0y, r0z;
     brick_centre(b, a.nb, a.bdim, a.nc, a.cs, r0x, r0y, r0z);
     const double us = TYPED ? 1.0 : a.inv_sigma;
-    for (int q = threadIdx.x; q < nh; q += blockDim.x) {
-        int gs;
-        double xx, yy, zz;
-        row_image(a.x, a.y, a.z, a.L[0], a.L[1], a.L[2], rows[q], gs, xx, yy, zz);
-        float4 v;
-        v.x = static_cast<float>((xx - r0x) * us);
-        v.y = static_cast<float>((yy - r0y) * us);
-        v.z = static_cast<float>((zz - r0z) * us);
-        v.w = TYPED ? __int_as_float(a.type[gs]) : 0.0f;
-        sp[q] = v;
+    // two threads per atom when the brick has at most half a block of atoms:
+    // lanes 2l and 2l+1 take alternate neighbour groups of atom l
+    const int tpa = (2 * nat <= kThreads) ? 2 : 1;
+    // (an empty brick may start past the last slot: its group loads read slot 0's)
+    const uint4* __restrict__ base = reinterpret_cast<const uint4*>(a.nbr16 + (int64_t)(nat > 0 ? a0 : 0) * a.cap);
+    int t = threadIdx.x;
+    AtomRow ar = atom_row(a.self16, a.numneigh, a0, nat, tpa, t);
+#pragma unroll
+    for (int k = 0; k < kHaloCap / kThreads; ++k) {
+        const int q = threadIdx.x + k * kThreads;
+        if (q < nh) {
+            int gs;
+            double xx, yy, zz;
+            row_image(a.x, a.y, a.z, a.L[0], a.L[1], a.L[2], row[k], gs, xx, yy, zz);
+            float4 v;
+            v.x = static_cast<float>((xx - r0x) * us);
+            v.y = static_cast<float>((yy - r0y) * us);
+            v.z = static_cast<float>((zz - r0z) * us);
+            v.w = TYPED ? __int_as_float(a.type[gs]) : 0.0f;
+            sp[q] = v;
+        }
     }
     if (threadIdx.x == 0) // the list's padding row: out of every cutoff
         sp[kSentinelRow] = make_float4(kSentinelFarF, kSentinelFarF, kSentinelFarF, __int_as_float(0));
+    uint4 s0 = base[group_at(ar, nat, 0, tpa)], s1 = base[group_at(ar, nat, 1, tpa)], s2;
     __syncthreads();
     const float rc_sq = static_cast<float>(a.rc_sq * us * us);
     const float eps4s = static_cast<float>(a.eps4), shifts = static_cast<float>(a.vshift);
     const float fscale = TYPED ? 1.0f : static_cast<float>(a.eps24 * a.inv_sigma);
     const double4* __restrict__ tab = a.tab;
     const int ntypes = a.ntypes;
-    const uint4* __restrict__ base = reinterpret_cast<const uint4*>(a.nbr16 + (int64_t)a0 * a.cap);
     // the cutoff decision inside the FP32 rounding band [rc_lo, rc_hi) around
     // rc^2 is the plain kernel's FP64 test on the same images: the main loop
     // counts the pairs below rc_lo and the fix-up below adds the band pairs the
@@ -409,19 +424,14 @@ __device__ void OpLjBrickMixed<EF, VF, TYPED>::run(const BrickLJArgs& a, int bid
     const double* __restrict__ gy = a.y;
     const double* __restrict__ gz = a.z;
     const double Lx = a.L[0], Ly = a.L[1], Lz = a.L[2];
-    // two threads per atom when the brick has at most half a block of atoms:
-    // lanes 2l and 2l+1 take alternate neighbour groups of atom l
-    const int tpa = (2 * nat <= static_cast<int>(blockDim.x)) ? 2 : 1;
-    for (int t = threadIdx.x; t < nat * tpa; t += blockDim.x) {
-        const int li = tpa == 2 ? (t >> 1) : t;
-        const int h = tpa == 2 ? (t & 1) : 0;
+    while (t < nat * tpa) {
+        const int li = ar.li, h = ar.h;
         const int i = a0 + li;
-        const int qs = a.self16[i];
+        const int qs = ar.qs;
         const float4 pi = sp[qs];
         const int ti = TYPED ? __float_as_int(pi.w) : 0;
-        const int nn = a.numneigh[i];
         const uint4* __restrict__ grp = base + li;
-        const int ng = (nn + kGroup - 1) / kGroup;
+        const int ng = ar.ng;
         float fxi = 0.f, fyi = 0.f, fzi = 0.f;
         bool near = false; // some pair's FP32 r^2 lies in [rc_lo, rc_hi)
         // group indices clamp to the last group (to group 0 when nn == 0: the
@@ -479,7 +489,6 @@ __device__ void OpLjBrickMixed<EF, VF, TYPED>::run(const BrickLJArgs& a, int bid
                 }
             }
         };
-        uint4 s0 = load(h), s1 = load(h + tpa), s2;
         for (int g = h;;) {
             if (g >= ng)
                 break;
@@ -559,11 +568,17 @@ __device__ void OpLjBrickMixed<EF, VF, TYPED>::run(const BrickLJArgs& a, int bid
             fyi += __shfl_xor(fyi, 1, 64);
             fzi += __shfl_xor(fzi, 1, 64);
         }
-        if (h != 0)
-            continue;
-        a.fx[i] = static_cast<double>(fxi * fscale);
-        a.fy[i] = static_cast<double>(fyi * fscale);
-        a.fz[i] = static_cast<double>(fzi * fscale);
+        if (h == 0) {
+            a.fx[i] = static_cast<double>(fxi * fscale);
+            a.fy[i] = static_cast<double>(fyi * fscale);
+            a.fz[i] = static_cast<double>(fzi * fscale);
+        }
+        t += kThreads;
+        if (t < nat * tpa) {
+            ar = atom_row(a.self16, a.numneigh, a0, nat, tpa, t);
+            s0 = base[group_at(ar, nat, 0, tpa)];
+            s1 = base[group_at(ar, nat, 1, tpa)];
+        }
     }
     if (EF || VF) {
         acc[0] *= 0.5;
