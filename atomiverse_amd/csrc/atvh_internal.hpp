@@ -269,8 +269,8 @@ inline int grid_capped(int64_t n, int block = kBlock) {
 
 // Pinned staging buffer of at least `bytes` (<= kPinMax); contents are the
 // caller's until its next stream synchronisation.
-constexpr size_t kPinMax = size_t(16) << 20;
-constexpr size_t kPinMin = size_t(256) << 10; // held from the context's creation
+constexpr size_t kPinMin = size_t(64) << 10; // held from the context's creation
+constexpr size_t kPinMax = size_t(2) << 20;  // taken at the first frame that needs more
 void* ctx_pin(atvh_ctx* c, size_t bytes);
 // The control block as of everything queued so far: one asynchronous copy into
 // pinned memory and one stream synchronisation.
@@ -284,7 +284,9 @@ struct HostPiece {
 // Frames of up to this many staged bytes travel through the context's pinned
 // buffer (one copy each way, one synchronisation); larger ones column by
 // column from and to the caller's memory, where the copy itself is the cost.
-constexpr size_t kStageMax = size_t(8) << 20;
+// (Pinning costs ~0.3 ms a MiB with its first touch: a 4 MiB buffer made a
+// context's first upload of 32,000 atoms 0.18 -> 1.2 ms.)
+constexpr size_t kStageMax = kPinMax;
 void fetch_pieces(atvh_ctx* c, const std::vector<HostPiece>& pieces);
 
 // Timing helpers (HIP events on the context stream, around one kernel family).

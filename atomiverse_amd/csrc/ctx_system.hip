@@ -51,9 +51,7 @@ void* ctx_pin(atvh_ctx* c, size_t bytes) {
             (void)hipHostFree(c->pin);
         c->pin = nullptr;
         c->pin_bytes = 0;
-        size_t want = kPinMin;
-        while (want < bytes)
-            want *= 2;
+        const size_t want = bytes <= kPinMin ? kPinMin : kPinMax;
         if (hipHostMalloc(&c->pin, want, hipHostMallocDefault) != hipSuccess) {
             c->pin = nullptr;
             throw Error(ATVH_E_NOMEM, "hipHostMalloc of the staging buffer failed");
