@@ -141,8 +141,18 @@ struct LjcArgs {
 // trajectory does not depend on which steps asked for energies.
 constexpr int kLjcLdsTypes = 4; // type tables up to this size are staged in LDS
 
-template <bool EF, bool VF, bool SMALLTAB>
-__global__ __launch_bounds__(kBlock) void k_ljc_brick_fp64(LjcArgs a) {
+// WIDE (at most kWideBricks bricks): twice the threads and up to four per atom.
+constexpr int kLjcFp64Threads = kBlock, kLjcFp64Wide = 512;
+
+// Threads per atom of a brick of nat atoms.
+template <bool WIDE>
+__device__ __forceinline__ int ljc_tpa(int nat, int threads) {
+    return WIDE && 4 * nat <= threads ? 4 : (2 * nat <= threads ? 2 : 1);
+}
+
+template <bool EF, bool VF, bool SMALLTAB, bool WIDE>
+__global__ __launch_bounds__(WIDE ? kLjcFp64Wide : kLjcFp64Threads) void k_ljc_brick_fp64(LjcArgs a) {
+    constexpr int kThreads = WIDE ? kLjcFp64Wide : kLjcFp64Threads;
     __shared__ double sx[kHaloCap], sy[kHaloCap], sz[kHaloCap], sq[kHaloCap];
     __shared__ int stype[kHaloCap];
     __shared__ double ljt[SMALLTAB ? kLjcLdsTypes * kLjcLdsTypes * 8 : 1]; // [ti][tj] lj1..lj4, shift
@@ -153,7 +163,7 @@ __global__ __launch_bounds__(kBlock) void k_ljc_brick_fp64(LjcArgs a) {
     double acc[7] = {0, 0, 0, 0, 0, 0, 0};
     if (brick_skipped(nh, nat, a.max_atoms)) { // reported by the build; nothing valid to compute
         if (EF || VF)
-            block_partials(acc, a.partials, blockIdx.x);
+            block_partials<kThreads>(acc, a.partials, blockIdx.x);
         return;
     }
     const int* __restrict__ rows = a.halo_rows + (int64_t)b * kHaloCap;
@@ -181,11 +191,10 @@ __global__ __launch_bounds__(kBlock) void k_ljc_brick_fp64(LjcArgs a) {
     const double* __restrict__ tab = a.tab;
     const double4* __restrict__ etab = a.erfc;
     const uint4* __restrict__ base = reinterpret_cast<const uint4*>(a.nbr16 + (int64_t)a0 * a.cap);
-    // two threads per atom when the brick has at most half a block of atoms
-    const int tpa = (2 * nat <= static_cast<int>(blockDim.x)) ? 2 : 1;
-    for (int t = threadIdx.x; t < nat * tpa; t += blockDim.x) {
-        const int li = tpa == 2 ? (t >> 1) : t;
-        const int h = tpa == 2 ? (t & 1) : 0;
+    const int tpa = ljc_tpa<WIDE>(nat, kThreads);
+    for (int t = threadIdx.x; t < nat * tpa; t += kThreads) {
+        const int li = t >> (tpa >> 1);
+        const int h = t & (tpa - 1);
         const int i = a0 + li;
         const int qs = a.self16[i];
         const double xi = sx[qs], yi = sy[qs], zi = sz[qs];
@@ -264,7 +273,12 @@ __global__ __launch_bounds__(kBlock) void k_ljc_brick_fp64(LjcArgs a) {
             cur = nx1;
             nx1 = nx2;
         }
-        if (tpa == 2) {
+        if (WIDE && tpa == 4) {
+            fxi += __shfl_xor(fxi, 2, 64);
+            fyi += __shfl_xor(fyi, 2, 64);
+            fzi += __shfl_xor(fzi, 2, 64);
+        }
+        if (tpa >= 2) {
             fxi += __shfl_xor(fxi, 1, 64);
             fyi += __shfl_xor(fyi, 1, 64);
             fzi += __shfl_xor(fzi, 1, 64);
@@ -279,7 +293,7 @@ __global__ __launch_bounds__(kBlock) void k_ljc_brick_fp64(LjcArgs a) {
 #pragma unroll
         for (int k = 0; k < 7; ++k)
             acc[k] *= 0.5; // full list: every pair seen from both ends
-        block_partials(acc, a.partials, blockIdx.x);
+        block_partials<kThreads>(acc, a.partials, blockIdx.x);
     }
 }
 
@@ -304,8 +318,10 @@ __device__ __forceinline__ float erfc_over_r(float x, float rinv, float& ex) {
 // force-only kernel (112 -> 107 us on the 512k-ion melt)
 constexpr int kLjcMixedThreads = 512;
 
-template <bool EF, bool VF, bool SMALLTAB>
-__global__ __launch_bounds__(kLjcMixedThreads) __attribute__((amdgpu_waves_per_eu((EF || VF) ? 4 : 8)))
+// WIDE: the same threads, up to four per atom, and the registers of the few
+// waves that are there.
+template <bool EF, bool VF, bool SMALLTAB, bool WIDE>
+__global__ __launch_bounds__(kLjcMixedThreads) __attribute__((amdgpu_waves_per_eu((EF || VF || WIDE) ? 4 : 8)))
 void k_ljc_brick_mixed(LjcArgs a) {
     __shared__ float4 sp[kHaloCap]; // x, y, z relative to the brick centre; w = charge
     __shared__ unsigned char stype[kHaloCap];
@@ -327,8 +343,7 @@ void k_ljc_brick_mixed(LjcArgs a) {
     }
     double r0x, r0y, r0z;
     brick_centre(b, a.nb, a.bdim, a.nc, a.cs, r0x, r0y, r0z);
-    // two threads per atom when the brick has at most half a block of atoms
-    const int tpa = (2 * nat <= kLjcMixedThreads) ? 2 : 1;
+    const int tpa = ljc_tpa<WIDE>(nat, kLjcMixedThreads);
     // (an empty brick may start past the last slot: its group loads read slot 0's)
     const uint4* __restrict__ base = reinterpret_cast<const uint4*>(a.nbr16 + (int64_t)(nat > 0 ? a0 : 0) * a.cap);
     int t = threadIdx.x;
@@ -431,7 +446,12 @@ void k_ljc_brick_mixed(LjcArgs a) {
             cur = nx1;
             nx1 = nx2;
         }
-        if (tpa == 2) {
+        if (WIDE && tpa == 4) {
+            fxi += __shfl_xor(fxi, 2, 64);
+            fyi += __shfl_xor(fyi, 2, 64);
+            fzi += __shfl_xor(fzi, 2, 64);
+        }
+        if (tpa >= 2) {
             fxi += __shfl_xor(fxi, 1, 64);
             fyi += __shfl_xor(fyi, 1, 64);
             fzi += __shfl_xor(fzi, 1, 64);
@@ -456,34 +476,43 @@ void k_ljc_brick_mixed(LjcArgs a) {
     }
 }
 
-template <bool SMALLTAB>
+template <bool SMALLTAB, bool WIDE>
 void launch_ljc_fp64(bool ef, bool vf, int grid, hipStream_t st, const LjcArgs& a) {
+    constexpr int nt = WIDE ? kLjcFp64Wide : kLjcFp64Threads;
     if (ef) {
         if (vf)
-            k_ljc_brick_fp64<true, true, SMALLTAB><<<grid, kBlock, 0, st>>>(a);
+            k_ljc_brick_fp64<true, true, SMALLTAB, WIDE><<<grid, nt, 0, st>>>(a);
         else
-            k_ljc_brick_fp64<true, false, SMALLTAB><<<grid, kBlock, 0, st>>>(a);
+            k_ljc_brick_fp64<true, false, SMALLTAB, WIDE><<<grid, nt, 0, st>>>(a);
     } else {
         if (vf)
-            k_ljc_brick_fp64<false, true, SMALLTAB><<<grid, kBlock, 0, st>>>(a);
+            k_ljc_brick_fp64<false, true, SMALLTAB, WIDE><<<grid, nt, 0, st>>>(a);
         else
-            k_ljc_brick_fp64<false, false, SMALLTAB><<<grid, kBlock, 0, st>>>(a);
+            k_ljc_brick_fp64<false, false, SMALLTAB, WIDE><<<grid, nt, 0, st>>>(a);
+    }
+}
+
+template <bool SMALLTAB, bool WIDE>
+void launch_ljc_mixed(bool ef, bool vf, int grid, hipStream_t st, const LjcArgs& a) {
+    if (ef) {
+        if (vf)
+            k_ljc_brick_mixed<true, true, SMALLTAB, WIDE><<<grid, kLjcMixedThreads, 0, st>>>(a);
+        else
+            k_ljc_brick_mixed<true, false, SMALLTAB, WIDE><<<grid, kLjcMixedThreads, 0, st>>>(a);
+    } else {
+        if (vf)
+            k_ljc_brick_mixed<false, true, SMALLTAB, WIDE><<<grid, kLjcMixedThreads, 0, st>>>(a);
+        else
+            k_ljc_brick_mixed<false, false, SMALLTAB, WIDE><<<grid, kLjcMixedThreads, 0, st>>>(a);
     }
 }
 
 template <bool SMALLTAB>
-void launch_ljc_mixed(bool ef, bool vf, int grid, hipStream_t st, const LjcArgs& a) {
-    if (ef) {
-        if (vf)
-            k_ljc_brick_mixed<true, true, SMALLTAB><<<grid, kLjcMixedThreads, 0, st>>>(a);
-        else
-            k_ljc_brick_mixed<true, false, SMALLTAB><<<grid, kLjcMixedThreads, 0, st>>>(a);
-    } else {
-        if (vf)
-            k_ljc_brick_mixed<false, true, SMALLTAB><<<grid, kLjcMixedThreads, 0, st>>>(a);
-        else
-            k_ljc_brick_mixed<false, false, SMALLTAB><<<grid, kLjcMixedThreads, 0, st>>>(a);
-    }
+void launch_ljc(bool mixed, bool wide, bool ef, bool vf, int grid, hipStream_t st, const LjcArgs& a) {
+    if (mixed)
+        wide ? launch_ljc_mixed<SMALLTAB, true>(ef, vf, grid, st, a) : launch_ljc_mixed<SMALLTAB, false>(ef, vf, grid, st, a);
+    else
+        wide ? launch_ljc_fp64<SMALLTAB, true>(ef, vf, grid, st, a) : launch_ljc_fp64<SMALLTAB, false>(ef, vf, grid, st, a);
 }
 
 // Small grids (< 2*reach+1 cells on an axis): global-slot ELL list with the
@@ -1283,16 +1312,11 @@ void ljc_enqueue(atvh_system* s, int precision, bool eflag, bool vflag) {
     hipStream_t st = s->ctx->stream;
     const int g = pair_grid(s);
     if (s->brick_mode) {
-        if (precision == ATVH_PREC_MIXED)
-            if (c->ntypes <= kLjcLdsTypes)
-                launch_ljc_mixed<true>(eflag, vflag, g, st, a);
-            else
-                launch_ljc_mixed<false>(eflag, vflag, g, st, a);
+        const bool mixed = precision == ATVH_PREC_MIXED, wide = s->nbricks <= kWideBricks;
+        if (c->ntypes <= kLjcLdsTypes)
+            launch_ljc<true>(mixed, wide, eflag, vflag, g, st, a);
         else
-            if (c->ntypes <= kLjcLdsTypes)
-                launch_ljc_fp64<true>(eflag, vflag, g, st, a);
-            else
-                launch_ljc_fp64<false>(eflag, vflag, g, st, a);
+            launch_ljc<false>(mixed, wide, eflag, vflag, g, st, a);
     } else {
         LJC_DISPATCH3(k_ljc_global, eflag, vflag, precision == ATVH_PREC_MIXED, g, st, a);
     }

@@ -112,14 +112,14 @@ struct AtomRow {
     int ng; // list groups
 };
 
-// Thread t's atom with tpa threads per atom (lanes 2l, 2l + 1 for tpa 2); a
+// Thread t's atom with tpa (1, 2 or 4) threads per atom in adjacent lanes; a
 // thread past the brick's atoms takes the last one's row header and uses none
 // of it.
 __device__ __forceinline__ AtomRow atom_row(const uint16_t* __restrict__ self16, const int* __restrict__ numneigh,
                                             int a0, int nat, int tpa, int t) {
     AtomRow r;
-    r.li = tpa == 2 ? (t >> 1) : t;
-    r.h = tpa == 2 ? (t & 1) : 0;
+    r.li = t >> (tpa >> 1);
+    r.h = t & (tpa - 1);
     r.qs = 0;
     r.ng = 0;
     if (r.li < nat) {
@@ -137,6 +137,11 @@ __device__ __forceinline__ AtomRow atom_row(const uint16_t* __restrict__ self16,
 __device__ __forceinline__ int group_at(const AtomRow& r, int nat, int k, int tpa) {
     return __umul24(min(r.h + k * tpa, max(r.ng - 1, 0)), nat) + r.li;
 }
+
+// Systems of at most this many bricks leave CUs with one workgroup or none, so
+// their force call is the latency of one brick: the wide kernels put more
+// threads on it. Beyond, workgroups share the CUs and the narrow ones win.
+constexpr int kWideBricks = 256; // one brick per CU
 
 // Small-grid pair kernels: kSmallLanes consecutive lanes share an atom, lane k
 // taking entries k, k + kSmallLanes, ... of its row. Those systems are a few

@@ -204,21 +204,44 @@ struct BrickLJArgs {
     double inv_sigma; // 1/sigma of the single-type form (coordinates in sigma units)
     float band;       // mixed: |r^2 - rc^2| below which the FP64 predicate decides (kernel units)
     int max_atoms;    // home atoms the list build took per brick
+    int wide;         // at most kWideBricks bricks: forces summed as four partials (OpLjFp64)
     const double4* tab;
     int ntypes;
     double *fx, *fy, *fz;
     double* partials;
 };
 
-template <bool EF, bool VF, bool TYPED>
-struct OpLjBrickFp64 {
+// A system of at most kWideBricks bricks (BrickLJArgs::wide) sums the force on
+// an atom in an order that does not depend on the threads: list group g belongs
+// to partial sum g mod 4, each partial adds its groups in list order, and the
+// total is (p0 + p2) + (p1 + p3). So one or two threads per atom (two partials
+// in each) and four give the same bits, and such a system alone runs the wide
+// form (500 atoms 8.7 -> 7.2 us, 4,000 atoms 13.5 -> 9.6) while a batch runs
+// the narrow one. Larger systems add their groups as they come: taking turns
+// between partials cost 5 us of 81 at 499,999 atoms.
+enum LjForm {
+    kLjPlain,  // narrow, larger systems
+    kLjEither, // narrow, by the system's size (batches; energy steps of small systems)
+    kLjWide,
+};
+
+template <bool EF, bool VF, bool TYPED, LjForm FORM>
+struct OpLjFp64 {
     using Args = BrickLJArgs;
-    static constexpr int kThreads = kBlock; // (512 measured slower: 311 vs 283 us at 2.048M atoms)
+    static constexpr bool WIDE = FORM == kLjWide;
+    static constexpr int kThreads = WIDE ? 1024 : kBlock; // narrow: 512 measured slower, 311 vs 283 us at 2.048M atoms
     static __device__ void run(const BrickLJArgs& a, int bid, int nbk);
 };
 
 template <bool EF, bool VF, bool TYPED>
-__device__ void OpLjBrickFp64<EF, VF, TYPED>::run(const BrickLJArgs& a, int bid, int nbk) {
+using OpLjBrickFp64 = OpLjFp64<EF, VF, TYPED, kLjPlain>;
+template <bool EF, bool VF, bool TYPED>
+using OpLjBrickFp64Either = OpLjFp64<EF, VF, TYPED, kLjEither>;
+template <bool EF, bool VF, bool TYPED>
+using OpLjBrickFp64Wide = OpLjFp64<EF, VF, TYPED, kLjWide>;
+
+template <bool EF, bool VF, bool TYPED, LjForm FORM>
+__device__ void OpLjFp64<EF, VF, TYPED, FORM>::run(const BrickLJArgs& a, int bid, int nbk) {
     __shared__ double sx[kHaloCap], sy[kHaloCap], sz[kHaloCap];
     __shared__ int stype[TYPED ? kHaloCap : 1];
     const int b = xcd_brick(bid, nbk); // one launch block per brick
@@ -255,12 +278,11 @@ __device__ void OpLjBrickFp64<EF, VF, TYPED>::run(const BrickLJArgs& a, int bid,
     const double4* __restrict__ tab = a.tab;
     const int ntypes = a.ntypes;
     const uint4* __restrict__ base = reinterpret_cast<const uint4*>(a.nbr16 + (int64_t)a0 * a.cap);
-    // two threads per atom when the brick has at most half a block of atoms:
-    // lanes 2l and 2l+1 take alternate neighbour groups of atom l
-    const int tpa = (2 * nat <= static_cast<int>(blockDim.x)) ? 2 : 1;
-    for (int t = threadIdx.x; t < nat * tpa; t += blockDim.x) {
-        const int li = tpa == 2 ? (t >> 1) : t;
-        const int h = tpa == 2 ? (t & 1) : 0;
+    // threads per atom, in adjacent lanes
+    const int tpa = WIDE && 4 * nat <= kThreads ? 4 : (2 * nat <= kThreads ? 2 : 1);
+    for (int t = threadIdx.x; t < nat * tpa; t += kThreads) {
+        const int li = t >> (tpa >> 1);
+        const int h = t & (tpa - 1);
         const int i = a0 + li;
         const int qs = a.self16[i];
         const double xi = sx[qs], yi = sy[qs], zi = sz[qs];
@@ -268,14 +290,11 @@ __device__ void OpLjBrickFp64<EF, VF, TYPED>::run(const BrickLJArgs& a, int bid,
         const int nn = a.numneigh[i];
         const uint4* __restrict__ grp = base + li;
         const int ng = (nn + kGroup - 1) / kGroup;
-        double fxi = 0.0, fyi = 0.0, fzi = 0.0;
         // group indices clamp to the last group (to group 0 when nn == 0: the
         // brick's rows always exist); loads run two groups ahead
         const int gl = max(ng - 1, 0);
-        uint4 cur = grp[__umul24(min(h, gl), nat)];
-        uint4 nx1 = grp[__umul24(min(h + tpa, gl), nat)];
-        for (int g = h; g < ng; g += tpa) {
-            const uint4 nx2 = grp[__umul24(min(g + 2 * tpa, gl), nat)];
+        auto load = [&](int g) { return grp[__umul24(min(g, gl), nat)]; };
+        auto group = [&](const uint4 cur, double3& f) {
             // the whole group's LDS reads issue before any arithmetic; padding
             // rows (the far sentinel) and pairs beyond r_c add zero
             const unsigned w[4] = {cur.x, cur.y, cur.z, cur.w};
@@ -308,9 +327,9 @@ __device__ void OpLjBrickFp64<EF, VF, TYPED>::run(const BrickLJArgs& a, int bid,
                 const double r2inv = 1.0 / r2;
                 const double r6inv = r2inv * r2inv * r2inv * sig6;
                 const double fpair = in ? eps24 * r2inv * fma(2.0 * r6inv, r6inv, -r6inv) : 0.0;
-                fxi = fma(fpair, dx, fxi);
-                fyi = fma(fpair, dy, fyi);
-                fzi = fma(fpair, dz, fzi);
+                f.x = fma(fpair, dx, f.x);
+                f.y = fma(fpair, dy, f.y);
+                f.z = fma(fpair, dz, f.z);
                 if (EF && in)
                     acc[0] += fma(eps4, r6inv * r6inv - r6inv, -shift);
                 if (VF && in) {
@@ -323,19 +342,58 @@ __device__ void OpLjBrickFp64<EF, VF, TYPED>::run(const BrickLJArgs& a, int bid,
                     acc[6] += dy * fzp;
                 }
             }
-            cur = nx1;
-            nx1 = nx2;
+        };
+        double3 f{0.0, 0.0, 0.0};
+        if (WIDE && tpa == 4) { // partial h
+            uint4 cur = load(h), nx1 = load(h + 4);
+#pragma unroll 1
+            for (int g = h; g < ng; g += 4) {
+                const uint4 nx2 = load(g + 8);
+                group(cur, f);
+                cur = nx1;
+                nx1 = nx2;
+            }
+            f.x += __shfl_xor(f.x, 2, 64);
+            f.y += __shfl_xor(f.y, 2, 64);
+            f.z += __shfl_xor(f.z, 2, 64);
+        } else if (FORM == kLjPlain || (FORM == kLjEither && !a.wide)) {
+            uint4 cur = load(h), nx1 = load(h + tpa);
+            for (int g = h; g < ng; g += tpa) {
+                const uint4 nx2 = load(g + 2 * tpa);
+                group(cur, f);
+                cur = nx1;
+                nx1 = nx2;
+            }
+        } else { // partials h and h + 2; with one thread per atom, then 1 and 3
+#pragma unroll 1
+            for (int hv = h; hv < 2; hv += tpa) {
+                double3 p{0.0, 0.0, 0.0}, q{0.0, 0.0, 0.0};
+                uint4 cur = load(hv), nx1 = load(hv + 2);
+#pragma unroll 1
+                for (int g = hv; g < ng; g += 2) {
+                    const uint4 nx2 = load(g + 4);
+                    group(cur, p);
+                    cur = nx1;
+                    nx1 = nx2;
+                    const double3 w = p; // the partials take turns (p + q does not depend on whose turn is last)
+                    p = q;
+                    q = w;
+                }
+                f.x = hv == h ? p.x + q.x : f.x + (p.x + q.x);
+                f.y = hv == h ? p.y + q.y : f.y + (p.y + q.y);
+                f.z = hv == h ? p.z + q.z : f.z + (p.z + q.z);
+            }
         }
-        if (tpa == 2) {
-            fxi += __shfl_xor(fxi, 1, 64);
-            fyi += __shfl_xor(fyi, 1, 64);
-            fzi += __shfl_xor(fzi, 1, 64);
+        if (tpa >= 2) {
+            f.x += __shfl_xor(f.x, 1, 64);
+            f.y += __shfl_xor(f.y, 1, 64);
+            f.z += __shfl_xor(f.z, 1, 64);
         }
         if (h != 0)
             continue;
-        a.fx[i] = fxi;
-        a.fy[i] = fyi;
-        a.fz[i] = fzi;
+        a.fx[i] = f.x;
+        a.fy[i] = f.y;
+        a.fz[i] = f.z;
     }
     if (EF || VF) {
 #pragma unroll
@@ -707,6 +765,7 @@ static BrickLJArgs brick_lj_args(atvh_system* s, const LJArgs& a) {
     b.numneigh = s->numneigh;
     b.cap = s->cap;
     b.max_atoms = brick_atom_limit(s);
+    b.wide = s->nbricks <= kWideBricks ? 1 : 0;
     for (int d = 0; d < 3; ++d) {
         b.L[d] = s->box[d];
         b.cs[d] = s->cs[d];
@@ -761,6 +820,12 @@ static void lj_enqueue(atvh_system* s, int precision, bool eflag, bool vflag) {
         atvh_ctx* c = s->ctx;
         if (precision == ATVH_PREC_MIXED)
             lj_brick_dispatch<OpLjBrickMixed>(c, eflag, vflag, typed, g, st, b);
+        else if (s->nbricks <= kWideBricks && (s->npt || !(eflag || vflag)))
+            // energies are summed thread by thread, so the steps of a run that
+            // a batch may also take keep the batch's narrow form for them
+            lj_brick_dispatch<OpLjBrickFp64Wide>(c, eflag, vflag, typed, g, st, b);
+        else if (s->nbricks <= kWideBricks)
+            lj_brick_dispatch<OpLjBrickFp64Either>(c, eflag, vflag, typed, g, st, b);
         else
             lj_brick_dispatch<OpLjBrickFp64>(c, eflag, vflag, typed, g, st, b);
         ATVH_HIP(hipGetLastError());
@@ -839,7 +904,7 @@ void pair_batch_launch(atvh_batch* b, int precision, bool ef, bool vf) {
     if (precision == ATVH_PREC_MIXED)
         pair_batch_dispatch<OpLjBrickMixed>(b, ef, vf);
     else
-        pair_batch_dispatch<OpLjBrickFp64>(b, ef, vf);
+        pair_batch_dispatch<OpLjBrickFp64Either>(b, ef, vf);
     ATVH_HIP(hipGetLastError());
 }
 
