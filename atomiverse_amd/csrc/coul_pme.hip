@@ -35,6 +35,9 @@
 //               energy and virial summed in FP64 over the half spectrum with
 //               the Hermitian partner of each interior mode folded in.
 //   5. hipFFT   C2R (Z2D / C2R).
+//               Steps 2-5 are three launches on meshes whose x-planes fit LDS
+//               (pme_plane.hpp) and five on larger FP32 power-of-two meshes
+//               (pme_fft.hpp); hipFFT takes the rest.
 //   6. gather   one thread per atom: weights and derivatives again, n^3 reads
 //               of the (L2-resident) grid,
 //               F = -(k_e / (pi V)) q sum_d g_d K_d / L_d, added to the forces.
@@ -44,6 +47,7 @@
 #include "brick.hpp"
 #include "pair_common.hpp"
 #include "pme_fft.hpp"
+#include "pme_plane.hpp"
 
 #include <hipfft/hipfft.h>
 
@@ -95,6 +99,11 @@ struct PmeState {
     // of PME at 128^3): twiddle tables exp(-2 pi i k / K_a), k <= K_a / 2
     bool native = false;
     float2* twf[3] = {nullptr, nullptr, nullptr};
+    // meshes whose planes fit LDS transform in three launches (pme_plane.hpp)
+    pmeplane::Axis axis[3];
+    bool plane32 = false, plane64 = false;
+    float2* ptw32[3] = {nullptr, nullptr, nullptr};
+    double2* ptw64[3] = {nullptr, nullptr, nullptr};
 };
 
 } // namespace atvh
@@ -1202,8 +1211,11 @@ void pme_release(PmeState* p) {
     dev_free(p->cplx32);
     dev_free(p->H);
     dev_free(p->partials);
-    for (int d = 0; d < 3; ++d)
+    for (int d = 0; d < 3; ++d) {
         dev_free(p->twf[d]);
+        dev_free(p->ptw32[d]);
+        dev_free(p->ptw64[d]);
+    }
     delete p;
 }
 
@@ -1336,15 +1348,37 @@ bool fft_native(const int K[3]) {
     return K[0] >= tile && K[0] <= maxk && K[1] >= tile && K[1] <= maxk && K[2] >= 2 * tile && K[2] <= 2 * maxk;
 }
 
-// Whether an evaluation of this precision runs the native transforms.
-bool pme_native(const PmeState* p, int precision) { return p->native && precision == ATVH_PREC_MIXED; }
+// Whether the three plane launches take this mesh with complex values of `cb`
+// bytes: a plane's two buffers and the tables fit LDS, and the radices cover
+// every axis of at most 128 points. Every such mesh that was measured against
+// the library's transforms gained (kernel time of unfix to inverse transform a
+// step, library -> planes): FP32 16^3 20 -> 18 us, 25^3 32 -> 19, 48^3 52 -> 26,
+// 96^3 59 -> 52, 108^3 64 -> 61, 120^3 101 -> 71; FP64 54^3 38 -> 35, 64^3
+// 39 -> 34, 80^3 45 -> 40, 90^3 68 -> 56. The five passes of pme_fft.hpp stay
+// ahead on their FP32 meshes, whose short tiles fill more CUs (32^3 19.5 us
+// against 22, 64^3 26 against 31, 128^3 56 against 72): they are asked first.
+bool plane_fits(const PmeState* p, size_t cb) {
+    const int K1 = p->K[1], K2 = p->K[2];
+    pmeplane::Axis t;
+    for (int d = 0; d < 3; ++d)
+        if (p->K[d] > pmeplane::kPlaneAxisMax || !pmeplane::make_axis(p->K[d], t))
+            return false;
+    const size_t plane = (2 * size_t(pmeplane::plane_values(K1, K2, p->Kh)) + K1 + K2) * cb;
+    return plane <= pmeplane::kPlaneLds && pmeplane::line_tiles(K1, p->Kh) <= kPmeGridCap;
+}
+bool pme_plane(const PmeState* p, int precision) { return precision == ATVH_PREC_MIXED ? p->plane32 : p->plane64; }
 
-// exp(-2 pi i k / L) for k = 0 .. L/2, from long double sin and cos.
+// Whether an evaluation of this precision runs the native transforms.
+bool pme_native(const PmeState* p, int precision) {
+    return p->native && precision == ATVH_PREC_MIXED;
+}
+
+// exp(-2 pi i k / L) for k = 0 .. n-1, from long double sin and cos.
 template <class T2, class T>
-T2* fft_twiddles(int L) {
-    std::vector<T2> h(L / 2 + 1);
+T2* fft_twiddles(int L, int n) {
+    std::vector<T2> h(n);
     const long double two_pi = 2.0L * std::acos(-1.0L);
-    for (int k = 0; k <= L / 2; ++k) {
+    for (int k = 0; k < n; ++k) {
         const long double ang = two_pi * static_cast<long double>(k) / static_cast<long double>(L);
         h[k].x = static_cast<T>(std::cos(ang));
         h[k].y = static_cast<T>(-std::sin(ang));
@@ -1440,6 +1474,8 @@ void fft_native_enqueue(atvh_system* s, const PmeArgs& pa, int ev, int gm, hipSt
 // Blocks (and fixed-order energy partials) of the influence kernel.
 int pme_grid_blocks(const atvh_system* s, int precision) {
     const PmeState* p = s->pme;
+    if (pme_plane(p, precision))
+        return pmeplane::line_tiles(p->K[1], p->Kh);
     if (pme_native(p, precision)) // pass C: one workgroup per tile, grid-stride beyond the partials' cap
         return std::min(p->K[1] * ((p->Kh - 1) / pmefft::kFftTile) + p->K[1] / pmefft::kFftTile, kPmeGridCap);
     const int64_t nmodes = (int64_t)p->K[0] * p->K[1] * p->Kh;
@@ -1451,12 +1487,27 @@ void pme_make_buffers(atvh_system* s, int precision) {
     PmeState* p = s->pme;
     const int64_t ntot = (int64_t)p->K[0] * p->K[1] * p->K[2];
     const int64_t nmodes = (int64_t)p->K[0] * p->K[1] * p->Kh;
+    if (pme_plane(p, precision)) {
+        if (precision == ATVH_PREC_MIXED && !p->real32) {
+            dev_alloc(&p->real32, ntot);
+            dev_alloc(&p->cplx32, nmodes);
+            for (int d = 0; d < 3; ++d)
+                p->ptw32[d] = fft_twiddles<float2, float>(p->K[d], p->K[d]);
+        }
+        if (precision != ATVH_PREC_MIXED && !p->real64) {
+            dev_alloc(&p->real64, ntot);
+            dev_alloc(&p->cplx64, nmodes);
+            for (int d = 0; d < 3; ++d)
+                p->ptw64[d] = fft_twiddles<double2, double>(p->K[d], p->K[d]);
+        }
+        return;
+    }
     if (pme_native(p, precision)) {
         if (!p->real32) {
             dev_alloc(&p->real32, ntot);
             dev_alloc(&p->cplx32, (int64_t)p->K[0] * p->K[1] * pmefft::fft_row(p->Kh));
             for (int d = 0; d < 3; ++d)
-                p->twf[d] = fft_twiddles<float2, float>(p->K[d]);
+                p->twf[d] = fft_twiddles<float2, float>(p->K[d], p->K[d] / 2 + 1);
         }
         return;
     }
@@ -1488,7 +1539,7 @@ void pme_prepare(atvh_system* s, int precision) {
     p->nb = pme_grid_blocks(s, precision);
     if (pme_ready(s, precision))
         return;
-    if (pme_native(p, precision)) { // nothing to load: the transforms are this library's kernels
+    if (pme_plane(p, precision) || pme_native(p, precision)) { // nothing to load: the transforms are this library's kernels
         pme_make_buffers(s, precision);
         p->nb = pme_grid_blocks(s, precision);
         return;
@@ -1513,6 +1564,45 @@ void pme_prepare(atvh_system* s, int precision) {
     if (free_before > free_after)
         note_fft_pair_bytes(static_cast<int64_t>(free_before - free_after));
     p->nb = pme_grid_blocks(s, precision);
+}
+
+// The three plane launches: fixed-point mesh in, real potential mesh out,
+// influence applied, energy (and virial) partials in gm blocks.
+template <class T, class T2>
+static void plane_enqueue(const PmeState* p, const PmeArgs& pa, T* real, T2* cplx, T2* const tw[3], int ev, int gm,
+                          hipStream_t st) {
+    using namespace pmeplane;
+    PlaneArgs f{};
+    f.a0 = p->axis[0];
+    f.a1 = p->axis[1];
+    f.a2 = p->axis[2];
+    f.Kh = p->Kh;
+    f.by2 = fast_div(p->K[2]);
+    f.byh = fast_div(p->Kh);
+    f.inv_fix = pa.inv_fix;
+    f.fix = p->fix;
+    f.real = real;
+    f.cplx = cplx;
+    f.tw0 = tw[0];
+    f.tw1 = tw[1];
+    f.tw2 = tw[2];
+    f.H = p->H;
+    f.ic0 = pa.ic0;
+    f.ic1 = pa.ic1;
+    f.ic2 = pa.ic2;
+    f.pi2_a2 = pa.pi2_a2;
+    f.partials = p->partials;
+    const size_t plds = (2 * size_t(plane_values(p->K[1], p->K[2], p->Kh)) + p->K[1] + p->K[2]) * sizeof(T2);
+    const size_t llds = (2 * size_t(kTile) * line_stride(p->K[0]) + p->K[0]) * sizeof(T2);
+    k_plane_forward<T><<<p->K[0], kPlaneThreads, plds, st>>>(f);
+    if (ev == 2)
+        k_lines_influence<T, 2><<<gm, kLineThreads, llds, st>>>(f);
+    else if (ev == 1)
+        k_lines_influence<T, 1><<<gm, kLineThreads, llds, st>>>(f);
+    else
+        k_lines_influence<T, 0><<<gm, kLineThreads, llds, st>>>(f);
+    k_plane_inverse<T><<<p->K[0], kPlaneThreads, plds, st>>>(f);
+    ATVH_HIP(hipGetLastError());
 }
 
 template <class T2>
@@ -1556,8 +1646,16 @@ void pme_enqueue(atvh_system* s, int precision, int ev) {
     }
     const int gg = grid_capped(ntot);
     const int gm = pme_grid_blocks(s, precision);
-    const bool native = pme_native(p, precision);
-    if (native) {
+    const bool plane = pme_plane(p, precision), native = plane || pme_native(p, precision);
+    if (plane && mixed) {
+        dispatch_order<float>(p->order, true, st, a, nullptr, sr);
+        plane_enqueue<float>(p, a, p->real32, p->cplx32, p->ptw32, ev, gm, st);
+        dispatch_order<float>(p->order, false, st, a, p->real32, sr);
+    } else if (plane) {
+        dispatch_order<double>(p->order, true, st, a, nullptr, sr);
+        plane_enqueue<double>(p, a, p->real64, p->cplx64, p->ptw64, ev, gm, st);
+        dispatch_order<double>(p->order, false, st, a, p->real64, sr);
+    } else if (native) {
         dispatch_order<float>(p->order, true, st, a, nullptr, sr);
         fft_native_enqueue<float>(s, a, ev, gm, st);
         dispatch_order<float>(p->order, false, st, a, p->real32, sr);
@@ -1605,10 +1703,13 @@ int64_t pme_device_bytes(const atvh_system* s) {
     const int64_t ntot = int64_t(p->K[0]) * p->K[1] * p->K[2];
     const int64_t nmodes = int64_t(p->K[0]) * p->K[1] * p->Kh;
     int64_t b = ntot * 8 + nmodes * 8 + int64_t(kPmeGridCap) * kPartialStride * 8; // fix, H, partials
+    const int64_t ptw = int64_t(p->K[0]) + p->K[1] + p->K[2]; // twiddles of the plane launches, no plans
     if (p->real64)
-        b += ntot * 8 + nmodes * 16 + fft_pair_bytes();
+        b += ntot * 8 + nmodes * 16 + (p->plane64 ? ptw * 16 : fft_pair_bytes());
     if (p->real32) {
-        if (p->native) // padded rows and three twiddle tables, no plans
+        if (p->plane32)
+            b += ntot * 4 + nmodes * 8 + ptw * 8;
+        else if (p->native) // padded rows and three twiddle tables, no plans
             b += ntot * 4 + int64_t(p->K[0]) * p->K[1] * pmefft::fft_row(p->Kh) * 8 +
                  int64_t(p->K[0] + p->K[1] + p->K[2] + 3) * 8;
         else
@@ -1799,6 +1900,10 @@ int atvh_pme_configure(atvh_system* s, double alpha, double spacing, int order) 
         }
         p->Kh = p->K[2] / 2 + 1;
         p->native = fft_native(p->K);
+        p->plane32 = !p->native && plane_fits(p, sizeof(float2));
+        p->plane64 = plane_fits(p, sizeof(double2));
+        for (int d = 0; d < 3; ++d)
+            pmeplane::make_axis(p->K[d], p->axis[d]);
         p->vol = s->box[0] * s->box[1] * s->box[2];
         const int64_t ntot = (int64_t)p->K[0] * p->K[1] * p->K[2];
         const int64_t nmodes = (int64_t)p->K[0] * p->K[1] * p->Kh;

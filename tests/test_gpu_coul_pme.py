@@ -155,6 +155,48 @@ def test_native_transform_meshes_match_oracle(hip_ctx, orc, K, order, stretch):
     assert s.energy()[0] == pe_m
 
 
+@pytest.mark.parametrize("mesh,order", [
+    ((25, 25, 25), 4),   # odd: the last packed pair of z-lines holds one line
+    ((27, 35, 30), 5),   # radices 3, 5, 7 and different axes
+    ((12, 49, 21), 4),   # 7 x 7, odd z
+    ((64, 20, 98), 6),   # power-of-two x in FP64, 2 x 7 x 7 z
+    ((14, 120, 18), 4),  # long y
+    ((12, 96, 100), 4),  # FP32 plane in LDS, FP64 plane over it
+    ((10, 135, 12), 4),  # an axis over the limit
+])
+def test_plane_transform_meshes_match_oracle(hip_ctx, orc, mesh, order):
+    """Meshes whose x-planes fit LDS transform in three launches; the bars are
+    those of the other meshes (same algorithm, transforms of the same
+    precision)."""
+    w = snapshot(12, seed=60 + order)
+    w.pme_order = order
+    f = np.array(mesh) / min(mesh)
+    h = w.box[0] / min(mesh)
+    w.box, w.x, w.y, w.z = w.box[0] * f, w.x * f[0], w.y * f[1], w.z * f[2]
+    w.pme_spacing = h * (1.0 + 1e-9)
+    s = make(hip_ctx, w)
+    Kd, _ = s.pme_info()
+    np.testing.assert_array_equal(Kd, mesh)
+    gx, gy, gz, e, ovir, parts = orc.pme(w.x, w.y, w.z, w.charge, w.box, w.alpha, Kd, order)
+    F = np.stack([gx, gy, gz])
+    s.pme_compute(av.PREC_FP64, True, True)
+    d = s.download()
+    pe, vir, _ = s.energy()
+    assert np.max(np.abs(forces(d) - F)) <= 1e-9 * np.max(np.abs(F))
+    assert pe == pytest.approx(e, rel=1e-9)
+    assert s.pme_info()[1][0] == pytest.approx(parts[0], rel=1e-9)
+    np.testing.assert_allclose(vir, ovir, rtol=1e-8, atol=1e-9 * np.abs(ovir[:3]).max())
+    s.pme_compute(av.PREC_MIXED, True, True)
+    m = s.download()
+    assert rms_rel(forces(m), F) <= 1e-5
+    pe_m, vir_m, _ = s.energy()
+    assert pe_m == pytest.approx(e, rel=1e-5)
+    assert np.linalg.norm(vir_m - ovir) <= 1e-5 * np.linalg.norm(ovir)
+    s.pme_compute(av.PREC_FP64, True, True)
+    assert s.energy()[0] == pe
+    np.testing.assert_array_equal(forces(s.download()), forces(d))
+
+
 def test_pme_is_bitwise_reproducible(hip_ctx):
     """Fixed-point spreading makes the charge grid independent of the order of
     the atomic adds: repeated evaluations agree bit for bit."""
