@@ -350,6 +350,8 @@ void nl_enqueue_pairs(atvh_system* s, const int* pred);
 // the permutation (from s->perm, keys in s->acell_of), halo tables and list
 // build after a sort that left the arrays in their old order
 void nl_enqueue_place(atvh_system* s);
+// the same after nl_enqueue_step_sort, which left a snapshot of the arrays
+void nl_enqueue_placed_lists(atvh_system* s);
 
 // pair_lj.hip
 int pair_grid(const atvh_system* s);

@@ -390,6 +390,20 @@ void md_enqueue_steps(atvh_system* s, int first, int nsteps, int precision, int 
         }
         return;
     }
+    if (large_step_fits(s)) {
+        for (int step = first; step < nsteps; ++step) {
+            if (!(resume && step == first))
+                large_enqueue_first_half(s, step > first ? step - 1 : -1, rec);
+            const bool ef = energy_step(step);
+            pair_enqueue(s, precision, ef, step == nsteps - 1);
+            if (ef)
+                energy_enqueue_finalize(s, rec_pe, step);
+            enqueue_final_kick(s, ia);
+        }
+        if (nsteps > first)
+            enqueue_final_post(s, nsteps - 1, rec);
+        return;
+    }
     PostArgs p_init = make_post_args(s, false, true);
     PostArgs p_fin = make_post_args(s, true, false);
     p_fin.record_ke = rec_ke;

@@ -103,19 +103,55 @@ __device__ __forceinline__ double nh_update(double ke, double dt, double ndof_kT
     return exp(-dt * 0.5 * xi);
 }
 
-// NeighborList::decide_reneighbor for this step (one thread).
-__device__ __forceinline__ bool decide_reneighbor(DevCtl* c, int every, int delay, int check, bool moved) {
-    const int ago = c->ago + 1;
-    const bool rb = ago >= delay && (ago % every) == 0 && (!check || moved);
-    c->disp_flag = 0;
+// NeighborList::decide_reneighbor, in the parts its callers order differently:
+// whether the list is due `ago` steps after its build, ...
+__device__ __forceinline__ bool reneighbor_due(int ago, int every, int delay, int check, bool moved) {
+    return ago >= delay && (ago % every) == 0 && (!check || moved);
+}
+// ... the decision as the rebuild stages read it (one thread) ...
+__device__ __forceinline__ void publish_rebuild(DevCtl* c, bool rb) {
     c->rebuild = rb ? 1 : 0;
-    c->ago = rb ? 0 : ago;
     if (rb) {
         c->nrebuilds += 1;
         c->nbr_total = 0;
         c->max_nbr = 0;
     }
+}
+// ... and the state the next decision reads (one thread).
+__device__ __forceinline__ void reneighbor_next(DevCtl* c, bool rb, int ago) {
+    c->disp_flag = 0;
+    c->ago = rb ? 0 : ago;
+}
+
+// NeighborList::decide_reneighbor for this step (one thread).
+__device__ __forceinline__ bool decide_reneighbor(DevCtl* c, int every, int delay, int check, bool moved) {
+    const int ago = c->ago + 1;
+    const bool rb = reneighbor_due(ago, every, delay, check, moved);
+    publish_rebuild(c, rb);
+    reneighbor_next(c, rb, ago);
     return rb;
+}
+
+// The NH half after the initial kick and the rebuild decision, for a launch
+// that finds both itself (k_step_bin).
+struct StepDecision {
+    DevCtl* ctl;
+    const double* partials; // m v^2 of the initial kick
+    int nb;
+    int thermostat;
+    double dt;
+    int every, delay, check;
+};
+
+// xi, scale and the half-step kinetic energy from the kick's total (one thread).
+__device__ __forceinline__ void initial_nh(const StepDecision& d, double mv2) {
+    DevCtl* c = d.ctl;
+    const double ke = 0.5 * mass_v2_to_energy * mv2;
+    double xi = c->xi_mid;
+    if (d.thermostat)
+        c->nh_scale = nh_update(ke, d.dt, c->nh_ndof_kT, c->nh_Q, xi);
+    c->xi = xi;
+    c->ke_half = ke;
 }
 
 struct FinalizeArgs {
@@ -160,6 +196,15 @@ __device__ __forceinline__ void finalize_totals(const FinalizeArgs& a) {
 void enqueue_final_kick(atvh_system* s, const IntArgs& a);
 void enqueue_final_post(atvh_system* s, int step, ThermoRec rec);
 double* ke_partials_of(const atvh_system* s, int which); // two sets of integ_grid partials
+
+// Launches of the multi-block steps (small_step.hip): the NH half of
+// final_step (< 0: none ends here), the next initial kick and drift, then the
+// decision and, on a rebuild, the sort and the lists.
+bool large_step_fits(const atvh_system* s);
+void large_enqueue_first_half(atvh_system* s, int final_step, ThermoRec rec);
+bool nl_step_sort_fits(const atvh_system* s); // neighbor.hip
+void nl_enqueue_step_sort(atvh_system* s, const StepDecision& d);
+int integ_grid(const atvh_system* s);
 
 IntArgs make_int_args(atvh_system* s);
 FinalizeArgs make_finalize_args(atvh_system* s, double* record_pe, int step, bool with_pair);

@@ -25,6 +25,7 @@
 #include "pair_common.hpp"
 
 #include <algorithm>
+#include <type_traits>
 
 using namespace atvh;
 
@@ -379,24 +380,29 @@ struct MidArgs {
     int step;
     BrickGeom g;
     double csx, csy, csz;
-    int* key; // cell rank of every slot at its new position
+    int* key; // cell rank of every slot at its new position (MID)
 };
 
 // The NH half of the step that ends (every block finds the same kinetic total
-// and scale; block 0 records), then kick, drift, displacement test and the
-// cell of every atom. xi and the scale are written by the next launch only:
-// blocks still read them here.
-__global__ __launch_bounds__(kBlock) void k_mid_initial(MidArgs a) {
+// and scale; block 0 records), then kick, drift, displacement test and, for the
+// mid path, the cell of every atom. xi and the scale are written by the next
+// launch only: blocks still read them here. A thread's first atom is loaded
+// ahead of the reduction.
+// MID: a thread per atom, with keys (as one kernel with a loop and a test for
+// the keys the mid path's launch took 0.4 us more of 5.3).
+template <bool MID>
+__global__ __launch_bounds__(kBlock) void k_step_initial(MidArgs a) {
     __shared__ double s_scale;
     DevCtl* c = a.i.ctl;
     const bool typed = a.i.ntypes > 1;
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    const bool act = i < static_cast<int>(a.i.n);
+    using Index = std::conditional_t<MID, int, int64_t>;
+    Index i = blockIdx.x * static_cast<Index>(kBlock) + threadIdx.x;
+    const Index stride = static_cast<Index>(gridDim.x) * kBlock;
     const int stop = c->overflow | c->halo_overflow;
     double scale = a.i.thermostat ? c->nh_scale : 1.0;
     KickAtom k{};
     double x[3] = {0, 0, 0}, xs[3] = {0, 0, 0};
-    if (act) {
+    const auto load = [&]() {
         k = kick_load(a.i, i, typed);
         x[0] = a.i.x[i];
         x[1] = a.i.y[i];
@@ -404,7 +410,10 @@ __global__ __launch_bounds__(kBlock) void k_mid_initial(MidArgs a) {
         xs[0] = a.i.xs[i];
         xs[1] = a.i.ys[i];
         xs[2] = a.i.zs[i];
-    }
+    };
+    const bool act = i < static_cast<Index>(a.i.n);
+    if (act)
+        load();
     if (stop)
         return;
     if (a.do_final) {
@@ -433,7 +442,7 @@ __global__ __launch_bounds__(kBlock) void k_mid_initial(MidArgs a) {
     }
     double mv2 = 0.0;
     bool moved = false;
-    if (act) {
+    const auto step = [&]() {
         mv2 += kick_apply(a.i, k, scale, typed, a.i.dtfm[0], a.i.mass[0]);
         x[0] = x[0] + a.i.dt * k.vx;
         x[1] = x[1] + a.i.dt * k.vy;
@@ -444,23 +453,26 @@ __global__ __launch_bounds__(kBlock) void k_mid_initial(MidArgs a) {
         a.i.vx[i] = k.vx;
         a.i.vy[i] = k.vy;
         a.i.vz[i] = k.vz;
-        moved = moved_past_skin(a.i, x[0] - xs[0], x[1] - xs[1], x[2] - xs[2]);
-        a.key[i] = a.g.cell_rank[bin_cell(a.i, a.g, a.csx, a.csy, a.csz, x)];
-    }
+        moved |= moved_past_skin(a.i, x[0] - xs[0], x[1] - xs[1], x[2] - xs[2]);
+        if (MID)
+            a.key[i] = a.g.cell_rank[bin_cell(a.i, a.g, a.csx, a.csy, a.csz, x)];
+    };
+    if (act)
+        step();
+    if (!MID)
+        for (i += stride; i < a.i.n; i += stride) {
+            load();
+            step();
+        }
     if (__any(moved) && (threadIdx.x & 63) == 0)
         c->disp_flag = 1;
     block_sum_to(mv2, &a.i.ke_partials[blockIdx.x]);
 }
 
 struct MidSortArgs {
-    DevCtl* ctl;
+    StepDecision d;
     FinalizeArgs e;
     int do_energy;
-    const double* partials; // m v^2 of the initial kick
-    int nb;
-    int thermostat;
-    double dt;
-    int every, delay, check;
     int n, ncells;
     const int* key;
     int* start; // [ncells + 1]
@@ -474,7 +486,7 @@ __global__ __launch_bounds__(kHeadThreads) void k_mid_sort(MidSortArgs a) {
     __shared__ int s_rebuild;
     __shared__ int s_wave[kHeadWaves];
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    DevCtl* c = a.ctl;
+    DevCtl* c = a.d.ctl;
     if (halted(c)) {
         if (tid == 0)
             c->rebuild = 0;
@@ -483,15 +495,10 @@ __global__ __launch_bounds__(kHeadThreads) void k_mid_sort(MidSortArgs a) {
     if (a.do_energy)
         finalize_totals(a.e);
     double sum[1];
-    block_fixed_sums<1>(a.partials, a.nb, 1, sum);
+    block_fixed_sums<1>(a.d.partials, a.d.nb, 1, sum);
     if (tid == 0) {
-        const double ke = 0.5 * mass_v2_to_energy * sum[0];
-        double xi = c->xi_mid;
-        if (a.thermostat)
-            c->nh_scale = nh_update(ke, a.dt, c->nh_ndof_kT, c->nh_Q, xi);
-        c->xi = xi;
-        c->ke_half = ke;
-        s_rebuild = decide_reneighbor(c, a.every, a.delay, a.check, c->disp_flag != 0) ? 1 : 0;
+        initial_nh(a.d, sum[0]);
+        s_rebuild = decide_reneighbor(c, a.d.every, a.d.delay, a.d.check, c->disp_flag != 0) ? 1 : 0;
     }
     __syncthreads();
     if (!s_rebuild)
@@ -578,36 +585,41 @@ bool mid_step_fits(const atvh_system* s) {
     return s->brick_mode && s->n <= kMidMaxAtoms && s->ncells < kMidMaxCells;
 }
 
+// The initial kick's launch (with the NH half of final_step); what the launch
+// after it needs to decide.
+static StepDecision enqueue_step_initial(atvh_system* s, int final_step, ThermoRec rec, int* key) {
+    ScopedTimer tm(s->ctx, "integrate");
+    MidArgs a{};
+    a.i = make_int_args(s);
+    a.final_partials = ke_partials_of(s, 0);
+    a.i.ke_partials = ke_partials_of(s, 1);
+    a.nb = integ_grid(s);
+    a.do_final = final_step >= 0 ? 1 : 0;
+    a.record_ke = rec.ke;
+    a.step = final_step;
+    a.g = brick_geom(s);
+    a.csx = s->cs[0];
+    a.csy = s->cs[1];
+    a.csz = s->cs[2];
+    a.key = key;
+    if (key) // n <= kMidMaxAtoms: integ_grid's cap is above that
+        k_step_initial<true><<<a.nb, kBlock, 0, s->ctx->stream>>>(a);
+    else
+        k_step_initial<false><<<a.nb, kBlock, 0, s->ctx->stream>>>(a);
+    ATVH_HIP(hipGetLastError());
+    return StepDecision{s->ctl, a.i.ke_partials, a.nb, s->thermostat, s->dt, s->every, s->delay, s->check};
+}
+
 void mid_enqueue_first_half(atvh_system* s, int final_step, bool final_energy, ThermoRec rec) {
     hipStream_t st = s->ctx->stream;
+    const StepDecision d = enqueue_step_initial(s, final_step, rec, s->acell_of);
     {
         ScopedTimer tm(s->ctx, "integrate");
-        MidArgs a{};
-        a.i = make_int_args(s);
-        a.final_partials = ke_partials_of(s, 0);
-        a.i.ke_partials = ke_partials_of(s, 1);
-        a.nb = grid_for(s->n);
-        a.do_final = final_step >= 0 ? 1 : 0;
-        a.record_ke = rec.ke;
-        a.step = final_step;
-        a.g = brick_geom(s);
-        a.csx = s->cs[0];
-        a.csy = s->cs[1];
-        a.csz = s->cs[2];
-        a.key = s->acell_of;
-        k_mid_initial<<<a.nb, kBlock, 0, st>>>(a);
         MidSortArgs m{};
-        m.ctl = s->ctl;
+        m.d = d;
         m.do_energy = final_step >= 0 && final_energy ? 1 : 0;
         if (m.do_energy)
             m.e = make_finalize_args(s, rec.pe, final_step, true);
-        m.partials = a.i.ke_partials;
-        m.nb = a.nb;
-        m.thermostat = s->thermostat;
-        m.dt = s->dt;
-        m.every = s->every;
-        m.delay = s->delay;
-        m.check = s->check;
         m.n = static_cast<int>(s->n);
         m.ncells = s->ncells;
         m.key = s->acell_of;
@@ -617,6 +629,19 @@ void mid_enqueue_first_half(atvh_system* s, int final_step, bool final_energy, T
         ATVH_HIP(hipGetLastError());
     }
     nl_enqueue_place(s);
+}
+
+// Larger systems sort over many blocks: eight launches a step (initial kick,
+// bin, scan, scatter, placement, list, forces, final kick) instead of twelve.
+// A launch that has nothing to do still takes 1.5-2 us of the stream, and on
+// nine steps of ten the rebuild's have nothing. The run's time a step: 499,999
+// atoms FP64 151 -> 144 us, 2,048,000 mixed 371 -> 363, melts of 110,592 ions
+// FP64 177 -> 170 and of 512,000 mixed 376 -> 366.
+bool large_step_fits(const atvh_system* s) { return s->brick_mode && nl_step_sort_fits(s); }
+
+void large_enqueue_first_half(atvh_system* s, int final_step, ThermoRec rec) {
+    nl_enqueue_step_sort(s, enqueue_step_initial(s, final_step, rec, nullptr));
+    nl_enqueue_placed_lists(s);
 }
 
 } // namespace atvh

@@ -1,8 +1,9 @@
 """The one-workgroup and few-launch steps of small systems against the
 multi-block stages, bit for bit: a system run alone (atvh_md_run picks the path
 by its size) equals the same system as the only member of a batch, which runs
-the multi-block stages. Sizes at the edges of the paths (1024, 2048 atoms, the
-cell limit of the sort), two types with charges and PME, a sparse box with more
+the multi-block stages. Sizes at the edges of the paths (1024, 2048 and 65,536
+atoms, the cell limit of the one-workgroup sort), more atoms than the kicks have
+threads, two types with charges and PME, a sparse box with more
 cells than the sort holds, an overflow halfway, and an odd cadence.
 """
 import numpy as np
@@ -49,13 +50,13 @@ def compare(ctx, w, steps, prec, every):
     s.close()
 
 
-@pytest.mark.parametrize("n", [500, 1024, 1025, 2048, 2049, 28000, 31500])
+@pytest.mark.parametrize("n", [500, 1024, 1025, 2048, 2049, 28000, 31500, 65537, 300001])
 @pytest.mark.parametrize("prec", [av.PREC_FP64, av.PREC_MIXED])
 def test_alone_equals_multi_block_stages(hip_ctx, n, prec):
     compare(hip_ctx, W.lj_trimmed(n, T_star=1.2, thermostat=n % 2), 60, prec, 7)
 
 
-@pytest.mark.parametrize("side", [10, 12, 14])
+@pytest.mark.parametrize("side", [10, 12, 14, 42])
 def test_charged_typed(hip_ctx, side):
     compare(hip_ctx, W.charged_melt(side, pme_spacing=1.0 / 1.2), 40, av.PREC_FP64, 7)
 
@@ -69,7 +70,7 @@ def test_cadence_and_sparse_box(hip_ctx):
     compare(hip_ctx, w, 60, av.PREC_FP64, 9)
 
 
-@pytest.mark.parametrize("n", [1372, 4000])
+@pytest.mark.parametrize("n", [1372, 4000, 70001])
 def test_overflow_halfway(hip_ctx, n):
     """A rebuild that overflows halts the run at its force phase; regrown and
     resumed there, it equals the run that never overflowed."""
