@@ -1,12 +1,12 @@
 // batch.hip — many independent systems advanced by one launch per stage.
 //
-// The step of every member is the single-system step (integrate.hip's fused
-// loop) with each stage launched once over all members: a member owns a
+// The step of every member is the single-system step's multi-block form
+// (a lone system takes fewer launches, small_step.hip) with each stage launched once over all members: a member owns a
 // contiguous range of the launch's blocks and runs exactly its own
 // single-system code on its own buffers (batch.hpp), so a member's trajectory
 // is bit-identical alone and in any batch. The per-step sequence — kick/drift,
-// NH + decide, the ten predicated rebuild stages, pair forces, energy totals,
-// final kick, NH + KE — is 16 or 17 launches whatever the number of members,
+// NH + decide, the active-member prefix and the seven predicated rebuild stages,
+// pair forces, energy totals, final kick, NH + KE — is 13 or 14 launches whatever the number of members,
 // and can be captured once into a hipGraph and replayed (no memset nodes: the
 // step clears its counters with kernels).
 //
