@@ -10,7 +10,8 @@
 // the second half of step k, the first half of step k + 1 and, when the list is
 // stale, the counting sort, the permutation and the halo tables are one launch
 // whose stages meet at workgroup barriers; the list build and the forces stay
-// one workgroup per brick. A step is three launches (500 atoms, FP64: 46 -> 19 us).
+// one workgroup per brick. A step is three launches (500 atoms, FP64: 46 -> 19
+// us, 17 with the wide force kernel).
 //
 // Every value is the multi-block stages' value bit for bit (the batched step
 // runs those, and a member equals the same system run alone): the per-atom
@@ -369,7 +370,8 @@ __global__ __launch_bounds__(kHeadThreads) void k_small_head(HeadArgs a) {
 // instead of a launch of its own; the decision and the sort's counting are one
 // workgroup, which needs only the 4-byte cell keys that kernel leaves; the
 // placement and the list build follow as two launches (nl_enqueue_place).
-// 32,000 atoms mixed 44.0 -> 37.1 us a step, 4,000 FP64 46 -> 31.
+// 32,000 atoms mixed 44.0 -> 37.1 us a step, 4,000 FP64 46 -> 31 (33.5 and 26.5
+// with the force kernels as they are now).
 
 struct MidArgs {
     IntArgs i;
