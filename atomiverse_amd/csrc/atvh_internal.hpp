@@ -239,7 +239,7 @@ struct atvh_batch {
     unsigned char* nl_flags = nullptr; // [nsys] this step's rebuild flags
     int* nl_next = nullptr;            // work counter of the pair-build stage (k_batched_queue)
     bool typed = false;
-    bool stages_changed = false; // some stage's tables were re-made (a captured step is stale)
+    bool stages_changed = false; // some stage's tables were re-made: set until the captured steps are dropped
     std::vector<int> nl_blocks;  // host copy of nl_nb
     // members whose force call is not the batched PairLJCut stage (charged
     // LJ + Coulomb with or without PME): queued one by one inside the step

@@ -149,13 +149,15 @@ void build_stages(atvh_batch* b, int nsteps) {
     }
     // stages whose members' arguments are unchanged keep their tables, and
     // the captured step stays valid with them; a step that queues a member's
-    // own force call captures that call's arguments, so it is captured anew
-    b->stages_changed = false;
+    // own force call captures that call's arguments, so it is captured anew.
+    // A builder that throws leaves stages_changed set: the captured steps point
+    // to tables that are gone, and the next build drops them
     integ_batch_build(b);
     nl_batch_build(b);
     pair_batch_build(b);
     if (b->stages_changed || !b->solo.empty())
         free_graphs(b);
+    b->stages_changed = false;
 }
 
 } // namespace

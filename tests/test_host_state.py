@@ -1,0 +1,30 @@
+"""What the library's host side keeps between calls (device tables, list rows,
+records, captured steps), on the stand-in HIP runtime: it must not outlive what
+it describes, whatever call failed in between."""
+from standin import standin  # noqa: F401
+
+MEMBERS = """
+ctx = av.Context(0)
+members = [make(ctx, W.lj_trimmed(n, thermostat=1)) for n in (500, 700)]
+b = av.Batch(ctx, members)
+b.set_graph(True)
+"""
+
+
+def test_refused_batch_run_leaves_no_captured_step(standin):  # noqa: F811
+    """A run that is refused after some stages were made anew (the longer record)
+    drops the captured steps: they point to the tables and records of before."""
+    standin(MEMBERS + """
+for _ in range(2):
+    b.run(50, energy_every=10)
+one = np.ones((2, 2))
+members[0].pair_lj(1.0, 1.0, 2.5, eps_tab=one, sigma_tab=one)
+try:
+    b.run(100, energy_every=10)
+    raise SystemExit("mixed single-type and per-type members were accepted")
+except av.HipError:
+    pass
+members[0].pair_lj(1.0, 1.0, 2.5)
+b.run(100, energy_every=10)
+assert hip.standin_stale() == 0, hip.standin_stale()
+""")
