@@ -438,7 +438,8 @@ namespace atvh {
 
 // The stage's device tables; a stage whose argument blocks and block counts
 // are those of the last run keeps them (a batch advances chunk after chunk
-// with unchanged members: re-making twelve stages took ~2 ms a run).
+// with unchanged members: re-making twelve stages took ~2 ms a run). The bytes
+// are compared, so blocks come zeroed, padding included.
 template <class Args>
 void batch_stage(atvh_batch* b, const std::string& name, const std::vector<Args>& args,
                  const std::vector<int>& blocks) {

@@ -2036,7 +2036,10 @@ void nl_batch_build(atvh_batch* b) {
         ba.push_back(nl_brick_args(s, pred));
         int gs[kNlStages + 1];
         nl_stage_grids(s, gs);
-        pa.push_back(PermHaloArgs{nl_perm_args(s, pred, false), ba.back(), gs[5]});
+        pa.emplace_back(); // zeroed, padding included: batch_stage compares bytes
+        pa.back().p = nl_perm_args(s, pred, false);
+        pa.back().h = ba.back();
+        pa.back().gp = gs[5];
         gs[5] += gs[6]; // the halo tables' blocks ride in the permutation's launch
         gs[6] = gs[7];
         for (int k = 0; k < kNlStages; ++k)

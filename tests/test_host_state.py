@@ -28,3 +28,16 @@ members[0].pair_lj(1.0, 1.0, 2.5)
 b.run(100, energy_every=10)
 assert hip.standin_stale() == 0, hip.standin_stale()
 """)
+
+
+def test_unchanged_batch_keeps_its_captured_steps(standin):  # noqa: F811
+    """A second run of unchanged members captures nothing: the bytes compared
+    are the arguments', padding included, so padding has to be defined."""
+    standin(MEMBERS + """
+b.run(20, energy_every=5)
+first = hip.standin_captures()
+assert first == 3 # forces, energies, the last step
+for _ in range(3):
+    b.run(20, energy_every=5)
+assert hip.standin_captures() == first, hip.standin_captures()
+""")
