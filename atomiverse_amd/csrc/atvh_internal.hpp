@@ -449,8 +449,8 @@ void batch_stage(atvh_batch* b, const std::string& name, const std::vector<Args>
     if (st.args && st.blocks == blocks && st.raw.size() == nraw && std::memcmp(st.raw.data(), raw, nraw) == 0)
         return;
     b->stages_changed = true;
-    st.raw.assign(raw, raw + nraw);
-    st.blocks = blocks;
+    st.blocks.clear(); // no key until the tables are whole: an allocation may fail below
+    st.raw.clear();
     dev_free(st.args);
     dev_free(st.base);
     dev_free(st.owner);
@@ -471,6 +471,8 @@ void batch_stage(atvh_batch* b, const std::string& name, const std::vector<Args>
     ATVH_HIP(hipMemcpy(st.base, base.data(), base.size() * sizeof(int), hipMemcpyHostToDevice));
     st.nblocks = base.back();
     st.nmembers = static_cast<int>(args.size());
+    st.raw.assign(raw, raw + nraw);
+    st.blocks = blocks;
 }
 
 } // namespace atvh

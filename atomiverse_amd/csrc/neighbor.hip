@@ -2058,7 +2058,7 @@ void nl_batch_build(atvh_batch* b) {
         nb.insert(nb.end(), g[k].begin(), g[k].end());
     if (b->nl_nb && nb == b->nl_blocks)
         return;
-    b->nl_blocks = nb;
+    b->nl_blocks.clear(); // no key until every table is whole
     b->stages_changed = true;
     dev_free(b->nl_nb);
     dev_free(b->nl_act);
@@ -2069,6 +2069,7 @@ void nl_batch_build(atvh_batch* b) {
     dev_alloc(&b->nl_flags, nsys);
     dev_alloc(&b->nl_next, 1);
     ATVH_HIP(hipMemcpy(b->nl_nb, nb.data(), nb.size() * sizeof(int), hipMemcpyHostToDevice));
+    b->nl_blocks = std::move(nb);
 }
 
 // This step's prefixes, per rebuild stage, of the block counts of the members

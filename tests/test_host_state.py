@@ -41,3 +41,47 @@ for _ in range(3):
     b.run(20, energy_every=5)
 assert hip.standin_captures() == first, hip.standin_captures()
 """)
+
+
+RETRY = """
+def retry(setup, call, close):
+    '''After each allocation of `call` that can fail, calling again leaves the
+    device memory that an undisturbed call leaves, and no launch on freed memory.'''
+    st = setup()
+    call(st)
+    want = live()
+    close(st)
+    st = setup()
+    failed = 0
+    for k in failing(lambda: call(st)):
+        call(st)
+        assert live() == want, (k, sum(live()) - sum(want))
+        assert hip.standin_stale() == 0, k
+        close(st)
+        st = setup()
+        failed += 1
+    close(st)
+    return failed
+
+def drop(st):
+    for o in reversed(st):
+        o.close()
+"""
+
+
+def test_batch_run_after_failed_allocation(standin):  # noqa: F811
+    standin(RETRY + """
+ctx = av.Context(0)
+
+def setup():
+    m = [make(ctx, W.lj_trimmed(n, thermostat=1)) for n in (500, 700)]
+    for s in m:
+        s.run(30) # lists and records are there
+    return m + [av.Batch(ctx, m)]
+
+for graph in (False, True):
+    def call(st):
+        st[-1].set_graph(graph)
+        st[-1].run(20)
+    assert retry(setup, call, drop) > 30
+""")
