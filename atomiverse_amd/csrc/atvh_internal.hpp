@@ -409,6 +409,7 @@ struct ThermoRec {
     double* ke;
 };
 ThermoRec thermo_rec(atvh_system* s); // the system's own per-step record
+void records_reserve(atvh_system* s, int nsteps); // ... of at least nsteps entries
 void md_enqueue_steps(atvh_system* s, int first, int nsteps, int precision, int energy_every, bool resume,
                       ThermoRec rec);
 // small_step.hip: whether one workgroup takes this system's integration and

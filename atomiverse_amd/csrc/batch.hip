@@ -136,12 +136,7 @@ void enqueue_step(atvh_batch* b, int precision, bool ef, bool vf) {
 void build_stages(atvh_batch* b, int nsteps) {
     // thermo buffers: one record per step per member, NaN where no energy was asked
     for (atvh_system* s : b->sys) {
-        if (s->thermo_cap < nsteps) {
-            dev_free(s->d_thermo);
-            s->thermo_cap = nsteps;
-            dev_alloc(&s->d_thermo, size_t(2) * nsteps);
-        }
-        s->thermo_n = nsteps;
+        records_reserve(s, nsteps);
         const int64_t nrec = int64_t(2) * s->thermo_cap;
         k_fill_nan<<<static_cast<int>(std::min<int64_t>((nrec + kBlock - 1) / kBlock, 1024)), kBlock, 0, b->ctx->stream>>>(
             s->d_thermo, nrec);

@@ -275,6 +275,16 @@ IntArgs make_int_args(atvh_system* s) {
     return a;
 }
 
+void records_reserve(atvh_system* s, int nsteps) {
+    if (s->thermo_cap < nsteps) {
+        s->thermo_n = s->thermo_cap = 0; // none, should the allocation fail
+        dev_free(s->d_thermo);
+        dev_alloc(&s->d_thermo, size_t(2) * nsteps);
+        s->thermo_cap = nsteps;
+    }
+    s->thermo_n = nsteps;
+}
+
 int integ_grid(const atvh_system* s) { return std::min(grid_for(s->n), kIntGrid); }
 
 void integ_enqueue_initial(atvh_system* s) {
@@ -637,12 +647,7 @@ int atvh_md_run(atvh_system* s, int nsteps, int precision, int energy_every) {
             return rc;
     }
     hipStream_t st = c->stream;
-    if (s->thermo_cap < nsteps) {
-        dev_free(s->d_thermo);
-        s->thermo_cap = nsteps;
-        dev_alloc(&s->d_thermo, size_t(2) * nsteps);
-    }
-    s->thermo_n = nsteps;
+    records_reserve(s, nsteps);
     if (s->npt) {
         // NoseHooverNPT: energies every step (its barostat reads the virial
         // and its conserved quantity the potential energy)

@@ -85,3 +85,18 @@ for graph in (False, True):
         st[-1].run(20)
     assert retry(setup, call, drop) > 30
 """)
+
+
+def test_records_after_failed_allocation(standin):  # noqa: F811
+    """The energy records of a longer run, alone and in a batch."""
+    standin(RETRY + """
+ctx = av.Context(0)
+
+def setup():
+    s = make(ctx, W.lj_trimmed(500, thermostat=1))
+    s.run(30)
+    return [s, av.Batch(ctx, [s])]
+
+for call in (lambda st: st[0].run(80), lambda st: st[1].run(80)):
+    assert retry(setup, call, drop) > 0
+""")
