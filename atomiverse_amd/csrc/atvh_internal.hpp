@@ -159,7 +159,7 @@ struct atvh_system {
     int* perm = nullptr;
     int* scan_sums = nullptr;
     int nscan_blocks = 0;
-    std::vector<int> nl_sig; // grid, bricks and stencil the list's tables were made for
+    std::vector<int> nl_sig; // grid, bricks and stencil the list's tables were made for (empty: not whole)
     int* nbr = nullptr;      // small-grid mode: ELL, column-major: nbr[k*npad + i]
     int* numneigh = nullptr; // [n]
     int cap = 0;

@@ -1494,17 +1494,25 @@ int64_t nl_device_bytes(const atvh_system* s) {
 }
 
 void nl_realloc_capacity(atvh_system* s, int cap) {
+    s->nl_built = false;
+    s->cap = 0; // no rows until they are there: the allocation may fail
     dev_free(s->nbr);
     dev_free(s->nbr16);
-    s->cap = (cap + 7) / 8 * 8;
+    cap = (cap + 7) / 8 * 8;
     if (s->brick_mode)
-        dev_alloc(&s->nbr16, size_t(s->cap) * s->n);
+        dev_alloc(&s->nbr16, size_t(cap) * s->n);
     else
-        dev_alloc(&s->nbr, size_t(s->cap) * s->npad);
+        dev_alloc(&s->nbr, size_t(cap) * s->npad);
+    s->cap = cap;
 }
 
-// CellList::compute_grid + build_stencil on the host (box-change only).
+// CellList::compute_grid + build_stencil on the host (box-change only). The
+// signature is empty from here until the tables are whole, so a call that
+// throws leaves no list and nl_build comes back here.
 void nl_setup_grid(atvh_system* s) {
+    std::vector<int> kept;
+    kept.swap(s->nl_sig);
+    s->nl_built = false;
     const double cutoff_skin = s->cutoff_skin;
     for (int d = 0; d < 3; ++d) {
         const double L = s->box[d];
@@ -1580,9 +1588,10 @@ void nl_setup_grid(atvh_system* s) {
         choose_bricks(s, s->brick_pick_min);
     sig.insert(sig.end(), {s->nc[0], s->nc[1], s->nc[2], s->reach[0], s->reach[1], s->reach[2],
                            s->brick_mode ? s->brick_pick : -1});
-    if (s->cell_rank && sig == s->nl_sig) {
+    if (sig == kept) {
         if (s->cap < cap)
             nl_realloc_capacity(s, cap);
+        s->nl_sig = std::move(kept);
         return;
     }
     nl_free(s);
@@ -1605,9 +1614,11 @@ void nl_setup_grid(atvh_system* s) {
     // per-block reduction partials: one row per pair workgroup (bricks) or grid block
     const int need = std::max(kMaxGrid, s->nbricks);
     if (need > s->npartials) {
+        double* p = nullptr;
+        dev_alloc(&p, size_t(2 * need) * kPartialStride); // pair | kinetic
         dev_free(s->partials);
+        s->partials = p;
         s->npartials = need;
-        dev_alloc(&s->partials, size_t(2 * s->npartials) * kPartialStride); // pair | kinetic
     }
     dev_alloc(&s->d_stencil, st.size());
     ATVH_HIP(hipMemcpy(s->d_stencil, st.data(), st.size() * sizeof(int), hipMemcpyHostToDevice));
@@ -1645,6 +1656,7 @@ void nl_setup_grid(atvh_system* s) {
 
 void nl_free(atvh_system* s) {
     s->nl_sig.clear();
+    s->cap = 0;
     dev_free(s->d_stencil);
     dev_free(s->halo_cells);
     dev_free(s->d_cols);
@@ -2164,6 +2176,8 @@ static void brick_fill(atvh_system* s, int& max_halo, int& max_atoms) {
 
 void nl_build(atvh_system* s, bool keep_counts) {
     atvh_ctx* c = s->ctx;
+    if (s->nl_sig.empty() || s->cap == 0) // an earlier allocation failed
+        nl_setup_grid(s);
     for (int attempt = 0; attempt < 12; ++attempt) {
         k_nl_stats_reset<<<1, 64, 0, c->stream>>>(s->ctl);
         // the initial build also orders the frame's forces (first kick uses them)
@@ -2270,7 +2284,6 @@ int atvh_nlist_set_capacity(atvh_system* s, int capacity) {
     ATVH_HIP(hipSetDevice(c->device));
     ATVH_HIP(hipStreamSynchronize(c->stream));
     nl_realloc_capacity(s, capacity);
-    s->nl_built = false;
     return ATVH_OK;
     API_CATCH(c)
 }

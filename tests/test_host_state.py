@@ -100,3 +100,65 @@ def setup():
 for call in (lambda st: st[0].run(80), lambda st: st[1].run(80)):
     assert retry(setup, call, drop) > 0
 """)
+
+
+def test_list_after_failed_allocation(standin):  # noqa: F811
+    """Grid tables and list rows: configured anew with the same and with other
+    cells, rows of another capacity, another brick shape."""
+    standin(RETRY + """
+ctx = av.Context(0)
+
+def setup():
+    s = make(ctx, W.lj_trimmed(500, thermostat=1))
+    s.run(30)
+    return [s]
+
+def same(st):
+    st[0].nlist_configure(2.5, 0.31)
+def more_rows(st):
+    st[0].nlist_configure(2.6, 0.3)
+def coarser(st):
+    st[0].nlist_configure(2.5, 0.6)
+def shape(st):
+    st[0].set_brick_shape(7)
+for change in (same, more_rows, coarser, shape):
+    def call(st):
+        change(st)
+        st[0].run(30)
+    assert retry(setup, call, drop) > 0 or change is same
+
+# the rows alone: whatever call comes next makes them again
+for after in (lambda s: s.run(30), lambda s: s.nlist_configure(2.5, 0.3), lambda s: s.nlist_build()):
+    [s] = setup()
+    want = live()
+    hip.standin_fail_after(0)
+    try:
+        s.set_capacity(400)
+        raise SystemExit("the allocation did not fail")
+    except av.HipError:
+        pass
+    hip.standin_fail_after(-1)
+    after(s)
+    assert live() == want, sum(live()) - sum(want)
+    s.close()
+""")
+
+
+def test_refused_grid_leaves_no_list(standin):  # noqa: F811
+    """A grid that is refused has replaced the cell sizes already: the list of
+    before is not run on."""
+    standin("""
+ctx = av.Context(0)
+s = make(ctx, W.lj_trimmed(500))
+s.run(5)
+for call in (lambda: s.nlist_configure(1e-3, 0.0), lambda: s.run(5), lambda: s.compute()):
+    n = hip.standin_launches()
+    try:
+        call()
+        raise SystemExit("accepted")
+    except av.HipError:
+        pass
+    assert hip.standin_launches() == n
+s.nlist_configure(2.5, 0.3)
+s.run(5)
+""")
