@@ -334,7 +334,7 @@ void dev_free(T*& p) {
 
 // neighbor.hip
 constexpr int kNlStages = 7; // kernels of one brick-mode rebuild
-void nl_setup_grid(atvh_system* s);
+void nl_setup_grid(atvh_system* s, bool keep_rows = false);
 void nl_enqueue_rebuild(atvh_system* s, const int* pred, bool permute_forces);
 void nl_enqueue_decide(atvh_system* s);
 void nl_free(atvh_system* s);

@@ -1508,8 +1508,9 @@ void nl_realloc_capacity(atvh_system* s, int cap) {
 
 // CellList::compute_grid + build_stencil on the host (box-change only). The
 // signature is empty from here until the tables are whole, so a call that
-// throws leaves no list and nl_build comes back here.
-void nl_setup_grid(atvh_system* s) {
+// throws leaves no list and nl_build comes back here. The rows take the
+// default capacity; keep_rows leaves longer ones while the tables stay.
+void nl_setup_grid(atvh_system* s, bool keep_rows) {
     std::vector<int> kept;
     kept.swap(s->nl_sig);
     s->nl_built = false;
@@ -1589,7 +1590,7 @@ void nl_setup_grid(atvh_system* s) {
     sig.insert(sig.end(), {s->nc[0], s->nc[1], s->nc[2], s->reach[0], s->reach[1], s->reach[2],
                            s->brick_mode ? s->brick_pick : -1});
     if (sig == kept) {
-        if (s->cap < cap)
+        if (keep_rows ? s->cap < cap : s->cap != cap)
             nl_realloc_capacity(s, cap);
         s->nl_sig = std::move(kept);
         return;

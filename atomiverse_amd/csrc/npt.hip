@@ -514,7 +514,7 @@ void npt_decide_rebuild(atvh_system* s, int& ago, int& nrebuilds) {
     if (!rebuild)
         return;
     if (stale)
-        nl_setup_grid(s); // CellList::compute_grid + build_stencil for the new box
+        nl_setup_grid(s, true); // CellList::compute_grid + build_stencil for the new box
     nl_build(s, true);    // records the box it was built in
     ago = 0;
     nrebuilds += 1;

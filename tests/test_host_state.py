@@ -162,3 +162,21 @@ for call in (lambda: s.nlist_configure(1e-3, 0.0), lambda: s.run(5), lambda: s.c
 s.nlist_configure(2.5, 0.3)
 s.run(5)
 """)
+
+
+def test_configure_restores_the_default_capacity(standin):  # noqa: F811
+    """A list set up again, also for the same cells and bricks, gives raised rows back."""
+    standin("""
+ctx = av.Context(0)
+s = make(ctx, W.lj_trimmed(500))
+s.run(5)
+cap, want = s.nlist_stats()["capacity"], live()
+for again in (lambda: s.nlist_configure(2.5, 0.3), lambda: s.set_brick_shape(s.brick_shape()[0])):
+    s.set_capacity(4 * cap)
+    s.run(5)
+    assert s.nlist_stats()["capacity"] == 4 * cap
+    again()
+    assert s.nlist_stats()["capacity"] == cap
+    s.run(5)
+    assert live() == want
+""")
