@@ -1482,47 +1482,42 @@ int pme_grid_blocks(const atvh_system* s, int precision) {
     return std::min(grid_for(nmodes), kPmeGridCap);
 }
 
-// The mesh buffers and transform plans of one precision.
-void pme_make_buffers(atvh_system* s, int precision) {
-    PmeState* p = s->pme;
+// The mesh buffers and transform plans of one precision. The real mesh is made
+// last: it says that the others are there (pme_ready), so what a call that
+// failed has left of them goes first.
+template <class T, class T2>
+void pme_make(PmeState* p, T*& real, T2*& cplx, T2* (&ptw)[3], bool plane, bool native, hipfftHandle& fwd,
+              hipfftHandle& back, hipfftType type_fwd, hipfftType type_back) {
+    if (real)
+        return;
     const int64_t ntot = (int64_t)p->K[0] * p->K[1] * p->K[2];
     const int64_t nmodes = (int64_t)p->K[0] * p->K[1] * p->Kh;
-    if (pme_plane(p, precision)) {
-        if (precision == ATVH_PREC_MIXED && !p->real32) {
-            dev_alloc(&p->real32, ntot);
-            dev_alloc(&p->cplx32, nmodes);
-            for (int d = 0; d < 3; ++d)
-                p->ptw32[d] = fft_twiddles<float2, float>(p->K[d], p->K[d]);
+    dev_free(cplx);
+    for (int d = 0; d < 3; ++d)
+        dev_free(ptw[d]);
+    for (hipfftHandle* h : {&fwd, &back})
+        if (*h) {
+            (void)hipfftDestroy(*h);
+            *h = nullptr;
         }
-        if (precision != ATVH_PREC_MIXED && !p->real64) {
-            dev_alloc(&p->real64, ntot);
-            dev_alloc(&p->cplx64, nmodes);
-            for (int d = 0; d < 3; ++d)
-                p->ptw64[d] = fft_twiddles<double2, double>(p->K[d], p->K[d]);
-        }
-        return;
+    dev_alloc(&cplx, native ? (int64_t)p->K[0] * p->K[1] * pmefft::fft_row(p->Kh) : nmodes);
+    if (plane || native) {
+        for (int d = 0; d < 3; ++d)
+            ptw[d] = fft_twiddles<T2, T>(p->K[d], plane ? p->K[d] : p->K[d] / 2 + 1);
+    } else {
+        HIPFFT_CHECK(hipfftPlan3d(&fwd, p->K[0], p->K[1], p->K[2], type_fwd));
+        HIPFFT_CHECK(hipfftPlan3d(&back, p->K[0], p->K[1], p->K[2], type_back));
     }
-    if (pme_native(p, precision)) {
-        if (!p->real32) {
-            dev_alloc(&p->real32, ntot);
-            dev_alloc(&p->cplx32, (int64_t)p->K[0] * p->K[1] * pmefft::fft_row(p->Kh));
-            for (int d = 0; d < 3; ++d)
-                p->twf[d] = fft_twiddles<float2, float>(p->K[d], p->K[d] / 2 + 1);
-        }
-        return;
-    }
-    if (precision == ATVH_PREC_MIXED && !p->real32) {
-        dev_alloc(&p->real32, ntot);
-        dev_alloc(&p->cplx32, nmodes);
-        HIPFFT_CHECK(hipfftPlan3d(&p->f32, p->K[0], p->K[1], p->K[2], HIPFFT_R2C));
-        HIPFFT_CHECK(hipfftPlan3d(&p->b32, p->K[0], p->K[1], p->K[2], HIPFFT_C2R));
-    }
-    if (precision != ATVH_PREC_MIXED && !p->real64) {
-        dev_alloc(&p->real64, ntot);
-        dev_alloc(&p->cplx64, nmodes);
-        HIPFFT_CHECK(hipfftPlan3d(&p->f64, p->K[0], p->K[1], p->K[2], HIPFFT_D2Z));
-        HIPFFT_CHECK(hipfftPlan3d(&p->b64, p->K[0], p->K[1], p->K[2], HIPFFT_Z2D));
-    }
+    dev_alloc(&real, ntot);
+}
+
+void pme_make_buffers(atvh_system* s, int precision) {
+    PmeState* p = s->pme;
+    if (precision == ATVH_PREC_MIXED)
+        pme_make(p, p->real32, p->cplx32, p->native ? p->twf : p->ptw32, p->plane32, p->native, p->f32, p->b32,
+                 HIPFFT_R2C, HIPFFT_C2R);
+    else
+        pme_make(p, p->real64, p->cplx64, p->ptw64, p->plane64, false, p->f64, p->b64, HIPFFT_D2Z, HIPFFT_Z2D);
 }
 
 // Everything a PME evaluation of this precision would allocate, made now:

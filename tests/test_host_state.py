@@ -180,3 +180,18 @@ for again in (lambda: s.nlist_configure(2.5, 0.3), lambda: s.set_brick_shape(s.b
     s.run(5)
     assert live() == want
 """)
+
+
+def test_mesh_after_failed_allocation(standin):  # noqa: F811
+    """Mesh buffers and twiddle tables of the plane transforms (both precisions)
+    and of the power-of-two ones."""
+    standin(RETRY + """
+ctx = av.Context(0)
+w25 = W.charged_melt(8, pme_spacing=1 / 1.2)
+w32 = W.charged_melt(8, pme_spacing=1.0)
+w32.pme_spacing = w32.box[0] / 31.9
+for w, prec in ((w25, av.PREC_FP64), (w25, av.PREC_MIXED), (w32, av.PREC_MIXED)):
+    assert retry(lambda: [make(ctx, w)], lambda st: st[0].run(10, prec), drop) > 4
+s = make(ctx, w32)
+assert s.pme_info()[0].tolist() == [32, 32, 32]
+""")
