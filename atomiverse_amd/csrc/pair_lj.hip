@@ -952,12 +952,7 @@ int atvh_pair_lj_configure(atvh_system* s, double eps, double sigma, double cuto
     if (ntypes > 0 && (!eps_tab || !sigma_tab))
         throw Error(ATVH_E_ARG, "PairLJCut: the per-type form needs eps and sigma tables");
     ATVH_HIP(hipSetDevice(c->device));
-    s->lj_eps = eps;
-    s->lj_sigma = sigma;
-    s->lj_cutoff = cutoff;
-    s->lj_ntypes = ntypes;
-    s->pair_style = 0;
-    dev_free(s->d_ljtab);
+    double* d_tab = nullptr;
     if (ntypes > 0) {
         // finalize_type_table_ (pair_lj_cut.cpp:257-298): sigma^6 and the
         // energy shift per pair; 24eps and 4eps prefactors.
@@ -973,10 +968,17 @@ int atvh_pair_lj_configure(atvh_system* s, double eps, double sigma, double cuto
             tab[4 * ab + 2] = s6;
             tab[4 * ab + 3] = 4.0 * e * (r6inv * r6inv - r6inv);
         }
-        dev_alloc(&s->d_ljtab, tab.size());
-        ATVH_HIP(hipMemcpy(s->d_ljtab, tab.data(), tab.size() * sizeof(double),
-                           hipMemcpyHostToDevice));
+        dev_alloc(&d_tab, tab.size());
+        ATVH_HIP(hipMemcpy(d_tab, tab.data(), tab.size() * sizeof(double), hipMemcpyHostToDevice));
     }
+    // the style changes once its table is there
+    dev_free(s->d_ljtab);
+    s->d_ljtab = d_tab;
+    s->lj_eps = eps;
+    s->lj_sigma = sigma;
+    s->lj_cutoff = cutoff;
+    s->lj_ntypes = ntypes;
+    s->pair_style = 0;
     s->pair_configured = true;
     return ATVH_OK;
     API_CATCH(c)

@@ -195,3 +195,26 @@ for w, prec in ((w25, av.PREC_FP64), (w25, av.PREC_MIXED), (w32, av.PREC_MIXED))
 s = make(ctx, w32)
 assert s.pme_info()[0].tolist() == [32, 32, 32]
 """)
+
+
+def test_pair_table_after_failed_allocation(standin):  # noqa: F811
+    """A per-type table that cannot be allocated leaves the pair style of before."""
+    standin("""
+ctx = av.Context(0)
+s = make(ctx, W.lj_trimmed(500))
+def table(n):
+    t = np.ones((n, n))
+    s.pair_lj(1.0, 1.0, 2.5, eps_tab=t, sigma_tab=t)
+table(2)
+s.run(5)
+want = live()
+hip.standin_fail_after(0)
+try:
+    table(3)
+    raise SystemExit("the allocation did not fail")
+except av.HipError:
+    pass
+hip.standin_fail_after(-1)
+assert live() == want
+s.run(5)
+""")
