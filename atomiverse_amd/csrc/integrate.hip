@@ -206,7 +206,13 @@ struct OpKinStressSum {
 
 struct OpFinalize {
     using Args = FinalizeArgs;
-    static __device__ void run(const FinalizeArgs& a, int, int) { finalize_totals(a); }
+    static __device__ void run(const FinalizeArgs& a, int, int) {
+        // a halted member of a batch stays at its step's record, which the run
+        // that goes on from there writes (or leaves empty)
+        if (a.step < 0 && halted(a.ctl))
+            return;
+        finalize_totals(a);
+    }
 };
 
 // Start of a fused run: no step of it completed yet.

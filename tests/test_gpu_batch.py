@@ -252,3 +252,33 @@ def test_batched_autotune_chooses_valid_shapes(hip_ctx):
             np.testing.assert_array_equal(d1[k], d0[k], err_msg=f"{w.name} {k}")
         s.close()
     b.close()
+
+
+@pytest.mark.parametrize("n", [1372, 4000])
+def test_records_of_a_member_halted_by_an_overflow(hip_ctx, n):
+    """A member halted by an overflow at a step without an energy request keeps
+    that step's record empty, whatever energy steps the batch takes before the
+    member goes on: its records are those of the run that never overflowed."""
+    every, nsteps = 50, 120
+    w = W.lj_trimmed(n, T_star=1.5, thermostat=1)
+    got = []
+    for tight in (False, True):
+        s = av.System(hip_ctx, w.n, w.box)
+        W.upload(s, w)
+        W.configure(s, w)
+        s.nlist_build()
+        if tight:
+            s.set_capacity(s.nlist_stats()["max_neighbors"])
+            s.nlist_build()
+            cap = s.nlist_stats()["capacity"]
+        b = av.Batch(hip_ctx, [s])
+        b.run(nsteps, av.PREC_FP64, energy_every=every)
+        got.append(s.thermo(nsteps))
+        if tight:
+            assert s.nlist_stats()["capacity"] > cap  # it did overflow
+        b.close()
+        s.close()
+    for a, b in zip(*got):
+        np.testing.assert_array_equal(b, a)
+    steps = np.flatnonzero(~np.isnan(got[0][0]))
+    np.testing.assert_array_equal(steps, [0, 50, 100, 119])
