@@ -282,3 +282,35 @@ def test_records_of_a_member_halted_by_an_overflow(hip_ctx, n):
         np.testing.assert_array_equal(b, a)
     steps = np.flatnonzero(~np.isnan(got[0][0]))
     np.testing.assert_array_equal(steps, [0, 50, 100, 119])
+
+
+def test_batch_goes_on_after_a_refused_run(hip_ctx):
+    """With captured steps: a run refused for mixed pair tables, after the longer
+    records were made, leaves nothing behind; set back, the batch equals one that
+    was never refused."""
+    one = np.ones((2, 2))
+    got = []
+    for refused in (False, True):
+        ms = members(hip_ctx, SIZES[:2])
+        b = av.Batch(hip_ctx, [s for _, s in ms])
+        b.set_graph(True)
+        for _ in range(2):
+            b.run(30, av.PREC_MIXED, energy_every=10)
+        if refused:
+            s = ms[0][1]
+            s.pair_lj(1.0, 1.0, 2.5, eps_tab=one, sigma_tab=one)
+            with pytest.raises(av.HipError):
+                b.run(60, av.PREC_MIXED, energy_every=10)
+            s.pair_lj(1.0, 1.0, 2.5)
+        for _ in range(2):
+            b.run(60, av.PREC_MIXED, energy_every=10)
+        got.append([snapshot(s, 60) for _, s in ms])
+        b.close()
+        for _, s in ms:
+            s.close()
+    for (d0, pe0, ke0, xi0, nr0), (d1, pe1, ke1, xi1, nr1) in zip(*got):
+        for k in d0:
+            np.testing.assert_array_equal(d1[k], d0[k])
+        np.testing.assert_array_equal(pe1, pe0)
+        np.testing.assert_array_equal(ke1, ke0)
+        assert xi1 == xi0 and nr1 == nr0
