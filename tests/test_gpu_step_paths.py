@@ -1,10 +1,11 @@
 """The one-workgroup and few-launch steps of small systems against the
 multi-block stages, bit for bit: a system run alone (atvh_md_run picks the path
 by its size) equals the same system as the only member of a batch, which runs
-the multi-block stages. Sizes at the edges of the paths (1024, 2048 and 65,536
-atoms, the cell limit of the one-workgroup sort), more atoms than the kicks have
-threads, two types with charges and PME, a sparse box with more
-cells than the sort holds, an overflow halfway, and an odd cadence.
+the multi-block stages. Sizes at the edges of the paths (1024 and 2048 atoms;
+EDGES: the atom and cell limits of the sorts), more atoms than the kicks have
+threads, two types with charges and PME in both precisions, a sparse box, an
+overflow halfway, and an odd cadence. That each size takes the path it stands for
+is checked on the CPU (test_host_state.py), by its launches a step.
 """
 import numpy as np
 import pytest
@@ -89,3 +90,34 @@ def test_overflow_halfway(hip_ctx, n):
         s.close()
     for a, b in zip(*got):
         np.testing.assert_array_equal(a, b)
+
+
+def stretched(n, z, cutoff=2.5):
+    """n atoms of the usual density in a box as long as z."""
+    w = W.lj_trimmed(n, T_star=1.2, thermostat=1)
+    w.box = np.array([w.box[0], w.box[1], max(z, w.box[2])])
+    w.cutoff = cutoff
+    return w
+
+
+# (workload, launches of a step): 3 up to 2,048 atoms while cells and atoms stay
+# under 14,000, 6 up to 65,536 atoms and 13,000 cells, else 8
+EDGES = {
+    "small": (lambda: stretched(700, 500.0), 3),                # 12,852 cells
+    "cells_over_small": (lambda: stretched(2000, 217.0), 6),    # 12,555 cells
+    "cells_over_both": (lambda: stretched(700, 525.0), 8),      # 13,500 cells
+    "atoms_at_mid": (lambda: stretched(65536, 0.0, 3.5), 6),    # 10,648 cells
+    "atoms_over_mid": (lambda: stretched(65537, 0.0, 3.5), 8),
+    "cells_under_mid": (lambda: stretched(31500, 0.0), 6),      # 12,167 cells
+    "cells_over_mid": (lambda: stretched(40000, 0.0), 8),       # 15,625 cells
+}
+
+
+@pytest.mark.parametrize("edge", sorted(EDGES))
+def test_alone_equals_multi_block_stages_at_the_edges(hip_ctx, edge):
+    compare(hip_ctx, EDGES[edge][0](), 60, av.PREC_FP64, 7)
+
+
+@pytest.mark.parametrize("side", [10, 12, 14, 42])
+def test_charged_typed_mixed(hip_ctx, side):
+    compare(hip_ctx, W.charged_melt(side, pme_spacing=1.0 / 1.2), 40, av.PREC_MIXED, 7)

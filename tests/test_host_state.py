@@ -218,3 +218,25 @@ hip.standin_fail_after(-1)
 assert live() == want
 s.run(5)
 """)
+
+
+def test_launches_of_a_step_by_size(standin):  # noqa: F811
+    """The path of each size in test_gpu_step_paths.py, by its launches a step."""
+    standin("""
+sys.path.insert(0, sys.argv[2] + "/tests")
+from test_gpu_step_paths import EDGES
+sizes = {k: v for k, v in EDGES.items()}
+for n, steps in ((500, 3), (1024, 3), (1025, 3), (2048, 3), (2049, 6), (28000, 6), (65537, 8)):
+    sizes[n] = (lambda n=n: W.lj_trimmed(n, T_star=1.2, thermostat=n % 2), steps)
+ctx = av.Context(0)
+for name, (workload, want) in sizes.items():
+    s = make(ctx, workload())
+    s.run(1)
+    count = []
+    for steps in (1, 11):
+        n = hip.standin_launches()
+        s.run(steps)
+        count.append(hip.standin_launches() - n)
+    assert (count[1] - count[0]) == 10 * want, (name, count)
+    s.close()
+""")
