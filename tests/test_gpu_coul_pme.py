@@ -328,3 +328,26 @@ def test_charged_errors(hip_ctx):
     with pytest.raises(av.HipError) as e:
         s.pme_compute()
     assert e.value.code == av._abi.E_STATE
+
+
+@pytest.mark.parametrize("mesh", [(25, 25, 25), (12, 49, 21), (12, 96, 100), (10, 135, 12), (32, 32, 32)])
+@pytest.mark.parametrize("prec", [av.PREC_FP64, av.PREC_MIXED])
+def test_energy_without_the_virial(hip_ctx, mesh, prec):
+    """An evaluation with the energy alone (what every energy step of a run but
+    the last asks for) gives the energy and forces of the one with the virial, bit
+    for bit, whichever kernels transform the mesh: the sums are the same sums."""
+    w = snapshot(12, seed=77)
+    f = np.array(mesh) / min(mesh)
+    h = w.box[0] / min(mesh)
+    w.box, w.x, w.y, w.z = w.box[0] * f, w.x * f[0], w.y * f[1], w.z * f[2]
+    w.pme_spacing = h * (1.0 + 1e-9)
+    s = make(hip_ctx, w)
+    np.testing.assert_array_equal(s.pme_info()[0], mesh)
+    got = []
+    for virial in (True, False):
+        s.pme_compute(prec, True, virial)
+        got.append((s.energy()[0], s.pme_info()[1], forces(s.download())))
+    for a, b in zip(*got):
+        np.testing.assert_array_equal(b, a)
+    assert got[0][0] != 0.0
+    s.close()
