@@ -140,7 +140,15 @@ __device__ __forceinline__ int group_at(const AtomRow& r, int nat, int k, int tp
 
 // Systems of at most this many bricks leave CUs with one workgroup or none, so
 // their force call is the latency of one brick: the wide kernels put more
-// threads on it. Beyond, workgroups share the CUs and the narrow ones win.
+// threads on it. Beyond, workgroups share the CUs, which the narrow ones do
+// better, the FP64 LJ + Coulomb kernel first. Launches, narrow / wide:
+//   FP64 LJ: 216 bricks 16.4 / 12.6 us, 252 24.7 / 15.9, 343 20.5 / 18.3,
+//   448 22.5 / 23.0, 640 37.7 / 37.7;
+//   FP64 LJ + Coulomb: 125 bricks 24.6 / 20.8, 288 25.5 / 27.2, 343 30.3 / 34.7,
+//   1,134 64 / 76;
+//   mixed LJ + Coulomb: 125 bricks 17.5 / 14.0, 288 19.2 / 16.1, 343 20.4 / 19.2,
+//   1,134 32.6 / 30.0.
+// One line for all, where none of them loses.
 constexpr int kWideBricks = 256; // one brick per CU
 
 // Small-grid pair kernels: kSmallLanes consecutive lanes share an atom, lane k

@@ -36,7 +36,7 @@ constexpr int kHeadThreads = 1024;
 constexpr int kHeadWaves = kHeadThreads / 64;
 constexpr int kHeadItems = 2; // most atoms per thread
 constexpr int kSmallMaxAtoms = kHeadThreads * kHeadItems;
-constexpr int kMidMaxAtoms = 65536;
+constexpr int kMidMaxAtoms = 45000;
 constexpr int kMidMaxCells = 13000;
 // cells + atoms the sort's LDS tables hold (start of every cell, tag of every slot)
 constexpr int kHeadLdsInts = 14000;
@@ -532,8 +532,10 @@ namespace atvh {
 // The line at kSmallMaxAtoms is one CU's memory path: at 4,000 atoms (four a
 // thread) this launch takes 20 us and a step 41 us, against 31 us with the
 // atoms spread over blocks (mid_enqueue_first_half); at 500 atoms it takes 5
-// us and a step 19 us (46 us with the multi-block stages). Cells count too: a
-// sparse box has more cells than the sort's LDS tables hold.
+// us and a step 19 us (46 us with the multi-block stages). Cells count too: the
+// sort's LDS tables hold kHeadLdsInts of them with the atoms, and a sparse box
+// gains little by then (700 atoms in 12,852 cells: a step 35 us, 32-36 us with
+// the atoms over blocks, 43 us beyond that form's lines).
 bool small_step_fits(const atvh_system* s) {
     return s->brick_mode && s->n <= kSmallMaxAtoms && s->ncells + s->n < kHeadLdsInts;
 }
@@ -581,8 +583,15 @@ void small_enqueue_head(atvh_system* s, int final_step, bool final_energy, bool 
     ATVH_HIP(hipGetLastError());
 }
 
-// Cells: the sort's LDS table (52 KB; a dense LJ fluid reaches it at 30,000
-// atoms). Atoms: one workgroup places them all.
+// One workgroup counts and places all keys, against a launch or two more that
+// spread the sort over the chip; us a step here / in large_enqueue_first_half:
+//   atoms, at few cells: 36,000 in 5,832 cells 61 / 60 FP64 and 63 / 63 mixed;
+//   50,000 in 8,000 82 / 79 and 73 / 70; 65,536 in 10,648 97 / 93 and 87 / 82.
+//   At cutoffs that make more cells of the same atoms the even point is higher
+//   (50,000 in 12,167 cells 57 / 57 and 48 / 51), so the line is between.
+//   cells, at the usual density: 31,500 atoms in 12,167 cells 37 / 41 and 39 / 44;
+//   40,000 in 15,625 47 / 51 and 44 / 47; 80,000 in 32,768 63 / 54 and 58 / 51.
+//   The table would fit LDS at any of these; the line is on the safe side.
 bool mid_step_fits(const atvh_system* s) {
     return s->brick_mode && s->n <= kMidMaxAtoms && s->ncells < kMidMaxCells;
 }

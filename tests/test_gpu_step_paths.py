@@ -101,13 +101,13 @@ def stretched(n, z, cutoff=2.5):
 
 
 # (workload, launches of a step): 3 up to 2,048 atoms while cells and atoms stay
-# under 14,000, 6 up to 65,536 atoms and 13,000 cells, else 8
+# under 14,000, 6 up to 45,000 atoms and 13,000 cells, else 8
 EDGES = {
     "small": (lambda: stretched(700, 500.0), 3),                # 12,852 cells
     "cells_over_small": (lambda: stretched(2000, 217.0), 6),    # 12,555 cells
     "cells_over_both": (lambda: stretched(700, 525.0), 8),      # 13,500 cells
-    "atoms_at_mid": (lambda: stretched(65536, 0.0, 3.5), 6),    # 10,648 cells
-    "atoms_over_mid": (lambda: stretched(65537, 0.0, 3.5), 8),
+    "atoms_at_mid": (lambda: stretched(45000, 0.0, 3.5), 6),    # 6,859 cells
+    "atoms_over_mid": (lambda: stretched(45001, 0.0, 3.5), 8),
     "cells_under_mid": (lambda: stretched(31500, 0.0), 6),      # 12,167 cells
     "cells_over_mid": (lambda: stretched(40000, 0.0), 8),       # 15,625 cells
 }
