@@ -355,7 +355,9 @@ void nl_enqueue_placed_lists(atvh_system* s);
 
 // pair_lj.hip
 int pair_grid(const atvh_system* s);
-void pair_enqueue(atvh_system* s, int precision, bool eflag, bool vflag);
+// in_run: a step of a run, whose virial nobody reads unless vflag; an evaluation
+// by itself that asks for the energy gets the k-space virial too
+void pair_enqueue(atvh_system* s, int precision, bool eflag, bool vflag, bool in_run = false);
 void pair_free(atvh_system* s);
 
 // coul_pme.hip

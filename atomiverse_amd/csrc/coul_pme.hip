@@ -1975,7 +1975,7 @@ int atvh_pme_compute(atvh_system* s, int precision, int eflag, int vflag) {
     ATVH_HIP(hipSetDevice(c->device));
     k_zero3<<<grid_capped(s->n), kBlock, 0, c->stream>>>(s->n, s->fx, s->fy, s->fz);
     ATVH_HIP(hipGetLastError());
-    const int ev = vflag ? 2 : (eflag ? 1 : 0);
+    const int ev = eflag || vflag ? 2 : 0;
     pme_enqueue(s, precision, ev);
     if (ev)
         energy_enqueue_finalize(s, nullptr, 0, false);

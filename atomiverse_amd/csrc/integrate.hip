@@ -387,7 +387,7 @@ void md_enqueue_steps(atvh_system* s, int first, int nsteps, int precision, int 
                 small_enqueue_head(s, step > first ? step - 1 : -1, energy_step(step - 1), true, rec);
                 nl_enqueue_pairs(s, &s->ctl->rebuild);
             }
-            pair_enqueue(s, precision, energy_step(step), step == nsteps - 1);
+            pair_enqueue(s, precision, energy_step(step), step == nsteps - 1, true);
         }
         if (nsteps > first)
             small_enqueue_head(s, nsteps - 1, true, false, rec);
@@ -397,7 +397,7 @@ void md_enqueue_steps(atvh_system* s, int first, int nsteps, int precision, int 
         for (int step = first; step < nsteps; ++step) {
             if (!(resume && step == first))
                 mid_enqueue_first_half(s, step > first ? step - 1 : -1, energy_step(step - 1), rec);
-            pair_enqueue(s, precision, energy_step(step), step == nsteps - 1);
+            pair_enqueue(s, precision, energy_step(step), step == nsteps - 1, true);
             enqueue_final_kick(s, ia);
         }
         if (nsteps > first) {
@@ -411,7 +411,7 @@ void md_enqueue_steps(atvh_system* s, int first, int nsteps, int precision, int 
             if (!(resume && step == first))
                 large_enqueue_first_half(s, step > first ? step - 1 : -1, rec);
             const bool ef = energy_step(step);
-            pair_enqueue(s, precision, ef, step == nsteps - 1);
+            pair_enqueue(s, precision, ef, step == nsteps - 1, true);
             if (ef)
                 energy_enqueue_finalize(s, rec_pe, step);
             enqueue_final_kick(s, ia);
@@ -435,7 +435,7 @@ void md_enqueue_steps(atvh_system* s, int first, int nsteps, int precision, int 
         }
         const bool ef = energy_step(step);
         // the virial is not recorded per step: only the last one can be read
-        pair_enqueue(s, precision, ef, step == nsteps - 1);
+        pair_enqueue(s, precision, ef, step == nsteps - 1, true);
         if (ef)
             energy_enqueue_finalize(s, rec_pe, step);
         {

@@ -701,7 +701,7 @@ static void lj_enqueue(atvh_system* s, int precision, bool eflag, bool vflag);
 // The force phase: the pair style (PairLJCut or PairLJCutCoulLong) writes the
 // forces, then KSpacePME adds its part when configured (the reference's
 // evaluator order at Phase::force).
-void pair_enqueue(atvh_system* s, int precision, bool eflag, bool vflag) {
+void pair_enqueue(atvh_system* s, int precision, bool eflag, bool vflag, bool in_run) {
     if (!s->pair_configured)
         throw Error(ATVH_E_STATE, "pair style not configured");
     if (!s->nl_built)
@@ -715,7 +715,7 @@ void pair_enqueue(atvh_system* s, int precision, bool eflag, bool vflag) {
         lj_enqueue(s, precision, eflag, vflag); // times its own launch
     }
     if (s->pme)
-        pme_enqueue(s, precision, vflag ? 2 : (eflag ? 1 : 0));
+        pme_enqueue(s, precision, vflag || (eflag && !in_run) ? 2 : (eflag ? 1 : 0));
 }
 
 static LJArgs lj_args(atvh_system* s) {
@@ -898,7 +898,7 @@ static void pair_batch_dispatch(atvh_batch* b, bool ef, bool vf) {
 
 void pair_batch_launch(atvh_batch* b, int precision, bool ef, bool vf) {
     for (atvh_system* s : b->solo)
-        pair_enqueue(s, precision, ef, vf);
+        pair_enqueue(s, precision, ef, vf, true);
     if (b->stages.find("pair") == b->stages.end())
         return;
     if (precision == ATVH_PREC_MIXED)

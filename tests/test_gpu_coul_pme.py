@@ -330,24 +330,45 @@ def test_charged_errors(hip_ctx):
     assert e.value.code == av._abi.E_STATE
 
 
-@pytest.mark.parametrize("mesh", [(25, 25, 25), (12, 49, 21), (12, 96, 100), (10, 135, 12), (32, 32, 32)])
-@pytest.mark.parametrize("prec", [av.PREC_FP64, av.PREC_MIXED])
-def test_energy_without_the_virial(hip_ctx, mesh, prec):
-    """An evaluation with the energy alone (what every energy step of a run but
-    the last asks for) gives the energy and forces of the one with the virial, bit
-    for bit, whichever kernels transform the mesh: the sums are the same sums."""
-    w = snapshot(12, seed=77)
+def stretched_snapshot(mesh, seed):
+    """The 1728-ion snapshot in a box whose sides go like the mesh's."""
+    w = snapshot(12, seed=seed)
     f = np.array(mesh) / min(mesh)
     h = w.box[0] / min(mesh)
     w.box, w.x, w.y, w.z = w.box[0] * f, w.x * f[0], w.y * f[1], w.z * f[2]
     w.pme_spacing = h * (1.0 + 1e-9)
+    return w
+
+
+@pytest.mark.parametrize("mesh", [(25, 25, 25), (12, 49, 21), (12, 96, 100), (10, 135, 12), (32, 32, 32)])
+@pytest.mark.parametrize("prec", [av.PREC_FP64, av.PREC_MIXED])
+def test_energy_steps_without_the_virial(hip_ctx, mesh, prec):
+    """An energy step of a run, which computes no virial, gives the energy that the
+    same step gives as the last one, which does, bit for bit, whichever kernels
+    transform the mesh: the sums are the same sums."""
+    w = stretched_snapshot(mesh, 77)
     s = make(hip_ctx, w)
     np.testing.assert_array_equal(s.pme_info()[0], mesh)
+    start = s.download()
+    got = []
+    for steps in (1, 2):
+        s.upload(start["x"], start["y"], start["z"], w.mass, w.vx, w.vy, w.vz, type_=w.type_, charge=w.charge)
+        s.run(steps, prec, energy_every=1)
+        got.append(s.thermo(1)[0][0])
+    assert got[0] == got[1] != 0.0
+    s.close()
+
+
+@pytest.mark.parametrize("mesh", [(25, 25, 25), (10, 135, 12), (32, 32, 32)])
+@pytest.mark.parametrize("prec", [av.PREC_FP64, av.PREC_MIXED])
+def test_evaluation_for_the_energy_has_the_kspace_virial(hip_ctx, mesh, prec):
+    """atvh_pme_compute with the energy alone answers as with both."""
+    s = make(hip_ctx, stretched_snapshot(mesh, 78))
     got = []
     for virial in (True, False):
         s.pme_compute(prec, True, virial)
-        got.append((s.energy()[0], s.pme_info()[1], forces(s.download())))
+        got.append((s.energy()[0], s.energy()[1], s.pme_info()[1], forces(s.download())))
     for a, b in zip(*got):
         np.testing.assert_array_equal(b, a)
-    assert got[0][0] != 0.0
+    assert np.abs(got[0][1][:3]).min() > 0.0
     s.close()
